@@ -316,6 +316,14 @@ int mykfa_validate_kv_append(const mykfa_kv_append_params* p);
 /* O and LSE (replaces _forward + _fwd_kernel, flash_attn.py:353-373, :106-154). */
 int mykfa_fwd(const mykfa_fwd_params* p, mykfa_stream_t stream);
 
+/* The same for dense layouts with few query blocks (a prompt of some hundred tokens behind a
+ * long cache): each block's keys are split over several workgroups, whose fp32 partials go to
+ * `workspace` (16-byte aligned, mykfa_fwd_workspace_size bytes) and are merged by a second
+ * launch. The size is 0 where the blocks alone fill the chip, and for packed layouts; the call
+ * is then mykfa_fwd (workspace may be NULL). */
+size_t mykfa_fwd_workspace_size(const mykfa_fwd_params* p);
+int mykfa_fwd_ws(const mykfa_fwd_params* p, void* workspace, size_t workspace_bytes, mykfa_stream_t stream);
+
 /* ---- backward ---------------------------------------------------------------------- */
 /* delta = rowsum(dO * O) in fp32 (the preprocess fused into _bwd_dq_kernel,
  * flash_attn.py:215-216). */

@@ -39,10 +39,44 @@ struct FwdArgs {
     int group;       // num_heads / num_kv_heads
     int hpw;         // query heads per workgroup
     int gx, gy, gz;  // query blocks, sequences, head groups; decoded by block_coord
+    // Key splits (SPLIT kernels): slots per block, and the fp32 partials of part = sequence *
+    // splits + split: unnormalized O [part][head][query][D], then (m, l) [part][head][query].
+    int splits;
+    float* ws_o;
+    f32x2* ws_ml;
 };
 
+// Tiles a key split holds at least: below it a part costs more in its prologue (Q rows and
+// first tiles landing, ~3 us) and in partials than its tiles take.
+constexpr int kMinSplitTiles = 4;
+
+// Key tiles [lo, lo + BN * n) of a workgroup's token blocks: the union over its tpw blocks of
+// 32 rows from tok_base.
+struct KeyTiles {
+    int lo, n;
+};
+__device__ inline KeyTiles key_tiles(int tok_base, int tpw, int q_len, int k_len, int lo_off, int hi_off, int BN) {
+    int wg_lo = 1 << 30, wg_hi = 0;
+    for (int tb = 0; tb < tpw; ++tb) {
+        int s0 = tok_base + tb * 32;
+        int bs = q_len - s0 < 32 ? q_len - s0 : 32;
+        if (bs <= 0) continue;
+        Ranges r = block_ranges(s0, bs, lo_off, hi_off, k_len, BN);
+        if (r.hi > r.lo) {
+            wg_lo = r.lo < wg_lo ? r.lo : wg_lo;
+            wg_hi = r.hi > wg_hi ? r.hi : wg_hi;
+        }
+    }
+    return KeyTiles{wg_lo, wg_hi > wg_lo ? (wg_hi - wg_lo + BN - 1) / BN : 0};
+}
+// Tiles per part of a block with n tiles and `splits` slots; it then has ceil(n / that) parts.
+__device__ inline int split_tiles(int n, int splits) {
+    const int t = (n + splits - 1) / splits;
+    return t < kMinSplitTiles ? kMinSplitTiles : t;
+}
+
 // Stage a BN x D tile (rows n0.., masked to < len) from global into a swizzled LDS tile.
-template <int D, int BN, int NW, int STAGES, typename T>
+template <int D, int BN, int NW, int STAGES, bool SPLIT, typename T>
 __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     constexpr int KD = D / 16;            // k-steps of S^T = K Q^T
     constexpr int DB = (D + 31) / 32;     // 32-row blocks of O^T
@@ -57,11 +91,15 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     const int tpw = NW / a.hpw;
     // Longest causal rows first across all heads and sequences (flash_attn.py:115 orders
     // within one head only), XCD-grouped.
-    const BlockCoord bc = block_coord(xcd_logical(__builtin_amdgcn_workgroup_id_x()), a.gz, a.gy, a.cu_q != nullptr);
+    // (The splits of a sequence count as further sequences: the query blocks that read the same
+    // keys then share an XCD's L2.)
+    const BlockCoord bc = block_coord(xcd_logical(__builtin_amdgcn_workgroup_id_x()), a.gz,
+                                      SPLIT ? a.gy * a.splits : a.gy, !SPLIT && a.cu_q != nullptr);
     if (bc.rank >= a.gx) return;
     const int mblk = a.gx - 1 - bc.rank;
     const int h_first = bc.group * a.hpw;
-    const int b = bc.seq;
+    const int b = SPLIT ? bc.seq / a.splits : bc.seq;
+    const int split = SPLIT ? bc.seq % a.splits : 0;
 
     SeqInfo qs = seq_info(b, a.cu_q, nullptr, a.seqlen_q, false);
     const int tok_base = mblk * tpw * 32;
@@ -72,17 +110,15 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     const int lo_off = band_lo(k_len, q_len, a.wl);
     const int hi_off = band_hi(k_len, q_len, a.wr);
 
-    // Key range of the workgroup: union over its token blocks.
-    int wg_lo = 1 << 30, wg_hi = 0;
-    for (int tb = 0; tb < tpw; ++tb) {
-        int s0 = tok_base + tb * 32;
-        int bs = q_len - s0 < 32 ? q_len - s0 : 32;
-        if (bs <= 0) continue;
-        Ranges r = block_ranges(s0, bs, lo_off, hi_off, k_len, BN);
-        if (r.hi > r.lo) {
-            wg_lo = r.lo < wg_lo ? r.lo : wg_lo;
-            wg_hi = r.hi > wg_hi ? r.hi : wg_hi;
-        }
+    // Key tiles of the workgroup; a split takes its run of them.
+    const KeyTiles all = key_tiles(tok_base, tpw, q_len, k_len, lo_off, hi_off, BN);
+    int wg_lo = all.lo, ntiles = all.n, parts = 1;
+    if constexpr (SPLIT) {
+        const int per = split_tiles(all.n, a.splits);
+        parts = all.n > per ? (all.n + per - 1) / per : 1;
+        if (split >= parts) return;
+        wg_lo += split * per * BN;
+        ntiles = min(per, all.n - split * per);
     }
 
     const int h = h_first + (wave % a.hpw);
@@ -96,7 +132,6 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     const i32x4 rsrc[2] = {rows_rsrc(kbase, k_len, a.kts, D), rows_rsrc(vbase, k_len, a.vts, D)};
     const int tstride[2] = {(int)(a.kts * 2), (int)(a.vts * 2)};
 
-    const int ntiles = wg_hi > wg_lo ? (wg_hi - wg_lo + BN - 1) / BN : 0;
     auto issue = [&](int t) {
         uint16_t* tiles[2] = {smem[t % STAGES][0], smem[t % STAGES][1]};
         Ring::issue(rsrc, tstride, tiles, wg_lo + t * BN, wave, lane);
@@ -259,6 +294,23 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     if (bs <= 0) return;
     // Epilogue (flash_attn.py:147-154): rows that saw no key output 0 and lse = +inf.
     const float l_tot = sum_halves(l_i);
+    if (SPLIT && parts > 1) {
+        // A part: O unnormalized and (m, l), all fp32, for merge_kernel.
+        if (qi < q_len) {
+            const int64_t row = ((int64_t)bc.seq * (a.gz * a.hpw) + h) * a.seqlen_q + qi;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int rq = 0; rq < 4; ++rq) {
+                    const int d0 = 32 * db + 8 * rq + 4 * g;
+                    if (d0 < D)
+                        *reinterpret_cast<f32x4*>(a.ws_o + row * D + d0) =
+                            f32x4{acc[db][4 * rq], acc[db][4 * rq + 1], acc[db][4 * rq + 2], acc[db][4 * rq + 3]};
+                }
+            if (g == 0) a.ws_ml[row] = f32x2{m_i, l_tot};
+        }
+        return;
+    }
     const bool empty = l_tot == 0.f;
     const float inv = empty ? 0.f : 1.f / l_tot;
     if (qi < q_len) {
@@ -278,6 +330,55 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     }
 }
 
+// O and LSE of the rows whose block ran in several parts (blocks of one part wrote theirs):
+// m = max m_s, l = sum l_s 2^(m_s - m), O = sum O_s 2^(m_s - m) / l, lse = m + log2 l. A row is
+// held by D / 4 lanes, 16 bytes of each part per lane, four parts in flight. Bound by the partials,
+// which the fp32 parts make 4 D + 8 bytes per row and part, mostly still in the caches.
+template <int D, int BN, typename T>
+__global__ __launch_bounds__(256) void merge_kernel(FwdArgs a, int tpw) {
+    constexpr int LPR = D / 4;  // lanes per row
+    const int heads = a.gz * a.hpw;
+    const int64_t idx = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;  // (sequence, query, head)
+    if (idx >= (int64_t)a.gy * a.seqlen_q * heads) return;
+    const int h = (int)(idx % heads), qi = (int)(idx / heads % a.seqlen_q), b = (int)(idx / heads / a.seqlen_q);
+    const SeqInfo ks = seq_info(b, nullptr, a.seqused_k, a.seqlen_k, true);
+    const int n = key_tiles(qi / (tpw * 32) * (tpw * 32), tpw, a.seqlen_q, ks.len, band_lo(ks.len, a.seqlen_q, a.wl),
+                            band_hi(ks.len, a.seqlen_q, a.wr), BN).n;
+    const int per = split_tiles(n, a.splits);
+    const int parts = n > per ? (n + per - 1) / per : 1;
+    if (parts == 1) return;
+    const int d0 = (threadIdx.x % LPR) * 4;
+    const int64_t row0 = ((int64_t)b * a.splits * heads + h) * a.seqlen_q + qi;
+    const int64_t ps = (int64_t)heads * a.seqlen_q;  // rows between consecutive parts
+    float m = kNegFloor, l = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < parts; s0 += 4) {
+        f32x2 ml[4];
+        f32x4 os[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int64_t row = row0 + min(s0 + u, parts - 1) * ps;
+            ml[u] = a.ws_ml[row];
+            os[u] = *reinterpret_cast<const f32x4*>(a.ws_o + row * D + d0);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (s0 + u >= parts) break;
+            const float mn = fmaxf(m, ml[u][0]);
+            const float w0 = fast_exp2(m - mn), w1 = fast_exp2(ml[u][0] - mn);
+            l = l * w0 + ml[u][1] * w1;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) o[c] = o[c] * w0 + os[u][c] * w1;
+            m = mn;
+        }
+    }
+    const bool empty = l == 0.f;
+    const float inv = empty ? 0.f : 1.f / l;
+    uint16_t* op = a.o + (int64_t)b * a.obs + (int64_t)qi * a.ots + (int64_t)h * a.ohs + d0;
+    *reinterpret_cast<u32x2*>(op) = u32x2{T::pack2(o[0] * inv, o[1] * inv), T::pack2(o[2] * inv, o[3] * inv)};
+    if (d0 == 0) a.lse[(int64_t)h * a.lse_hs + (int64_t)b * a.seqlen_q + qi] = empty ? INFINITY : m + fast_log2(l);
+}
+
 int gcd_int(int x, int y) {
     while (y) {
         int t = x % y;
@@ -294,10 +395,20 @@ hipError_t launch_typed(FwdArgs args, int batch, int num_heads, int max_q, hipSt
     args.gx = (max_q + tpw * 32 - 1) / (tpw * 32);
     args.gy = batch;
     args.gz = num_heads / args.hpw;
-    const long long n = block_grid_size(args.gx, args.gz, args.gy, args.cu_q != nullptr);
+    const int slots = args.splits > 1 ? args.splits : 1;
+    const long long n = block_grid_size(args.gx, args.gz, args.gy * slots, args.cu_q != nullptr);
     if (n == 0) return hipSuccess;
     if (n > (1LL << 30)) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((fwd_kernel<D, BN, NW, STAGES, T>), dim3(xcd_grid((int)n)), dim3(NW * 64), 0, s, args);
+    if (args.splits <= 1) {
+        hipLaunchKernelGGL((fwd_kernel<D, BN, NW, STAGES, false, T>), dim3(xcd_grid((int)n)), dim3(NW * 64), 0, s, args);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL((fwd_kernel<D, BN, NW, STAGES, true, T>), dim3(xcd_grid((int)n)), dim3(NW * 64), 0, s, args);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const long long rows = (long long)batch * max_q * num_heads;
+    constexpr int RPB = 256 / (D / 4);
+    hipLaunchKernelGGL((merge_kernel<D, BN, T>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, s, args, tpw);
     return hipGetLastError();
 }
 
@@ -320,8 +431,38 @@ hipError_t launch_dtype(const FwdArgs& args, int D, int batch, int num_heads, in
 
 }  // namespace
 
-hipError_t launch_fwd(const mykfa_fwd_params& p, hipStream_t stream) {
+size_t fwd_split_bytes(const mykfa_fwd_params& p, int splits) {
+    if (splits <= 1) return 0;
+    return (size_t)splits * p.batch * p.num_heads * p.max_seqlen_q * ((size_t)p.head_dim + 2) * sizeof(float);
+}
+
+// Parts per block when the blocks alone leave CUs idle (a prompt of some hundred tokens behind a
+// long cache: 389 queries of 16 heads are 52 workgroups of 100 key tiles each, 112.7 us on 256
+// CUs). Parts up to one workgroup per CU: measured (us, at 1 / 128 / 192 / 256 / 384 / 512 / 1024
+// workgroups) 112.7 / 66.7 / 50.7 / 45.4 / 42.3 / 51.4 / 59.4 there (bf16, D 128, 6389 keys),
+// 71.4 / 47.6 / 40.6 / 37.7 / 37.5 / 36.4 / 47.4 with 1000 queries of 8 heads on 3000 keys, 44.7 / 44.3 /
+// 32.6 / 32.5 / 30.1 / 31.3 / 34.6 with 2 x 1500 queries of 4 heads of 64 on 2000 keys: beyond one
+// workgroup per CU the partials cost what the shorter chains save. A block whose keys could fill
+// fewer than 16 tiles is not split: a 512 window took 18.4 us whole and 21.7 in two parts.
+int fwd_default_splits(const mykfa_fwd_params& p) {
+    if (p.cu_seqlens_q != nullptr || p.batch <= 0 || p.max_seqlen_q <= 0) return 1;
+    const int hpw = gcd_int(p.num_heads / p.num_kv_heads, 4), rows = 4 / hpw * 32, BN = p.head_dim > 128 ? 32 : 64;
+    const long long blocks = (long long)p.batch * (p.num_heads / hpw) * ((p.max_seqlen_q + rows - 1) / rows);
+    long long span = (long long)p.window_left + p.window_right + rows + BN;  // most keys a block sees
+    if (span > p.max_seqlen_k) span = p.max_seqlen_k;
+    const long long tiles = (span + BN - 1) / BN;
+    long long splits = 256 / blocks;
+    if (splits > tiles / 8) splits = tiles / 8;
+    if (splits > 64) splits = 64;
+    return splits < 2 ? 1 : (int)splits;
+}
+
+hipError_t launch_fwd(const mykfa_fwd_params& p, int splits, void* ws, hipStream_t stream) {
     FwdArgs a;
+    a.splits = splits;
+    a.ws_o = static_cast<float*>(ws);
+    a.ws_ml = splits > 1 ? reinterpret_cast<f32x2*>(a.ws_o + (size_t)splits * p.batch * p.num_heads * p.max_seqlen_q * p.head_dim)
+                         : nullptr;
     a.q = static_cast<const uint16_t*>(p.q);
     a.k = static_cast<const uint16_t*>(p.k);
     a.v = static_cast<const uint16_t*>(p.v);

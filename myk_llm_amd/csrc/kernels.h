@@ -8,7 +8,12 @@
 
 namespace mykfa {
 
-hipError_t launch_fwd(const mykfa_fwd_params& p, hipStream_t stream);
+// Prefill forward. With splits > 1 (dense layouts) each block's keys go in up to `splits` parts,
+// fp32 partials in ws (fwd_split_bytes) and a merge; fwd_default_splits: 1 unless the blocks
+// alone leave the chip idle.
+int fwd_default_splits(const mykfa_fwd_params& p);
+size_t fwd_split_bytes(const mykfa_fwd_params& p, int splits);
+hipError_t launch_fwd(const mykfa_fwd_params& p, int splits, void* ws, hipStream_t stream);
 
 hipError_t launch_bwd_preprocess(const mykfa_bwd_params& p, hipStream_t stream);
 hipError_t launch_bwd_dkdv(const mykfa_bwd_params& p, hipStream_t stream);

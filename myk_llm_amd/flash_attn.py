@@ -43,6 +43,9 @@ from . import _lib
 _UNBOUNDED = _lib.UNBOUNDED  # flash_attn.py:32
 _HEAD_DIMS = (16, 32, 64, 128, 256)  # flash_attn.py:322-323
 _DECODE_MAX_Q = 16  # few queries per sequence use the split-K decode kernel (flash_attn.py:364)
+# Only batches of at most this many (query, head) rows can have their keys split by the forward:
+# 128 rows a workgroup, at least two parts for each of the 256 CUs' workgroups.
+_SPLIT_MAX_ROWS = 128 * 128
 
 
 def _ds_budget_bytes() -> int:
@@ -237,6 +240,11 @@ def _forward(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Optional[Tensor], cu
     with _DeviceGuard(dev):
         if not varlen and 0 < max_seqlen_q <= _DECODE_MAX_Q:
             _decode_launch(L, p, dev)
+        elif (not varlen and shape[0] * shape[1] * shape[2] <= _SPLIT_MAX_ROWS
+              and (nbytes := L.mykfa_fwd_workspace_size(ctypes.byref(p)))):
+            # Too few query blocks to fill the chip: their keys are split, partials merged.
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            _lib.check(L.mykfa_fwd_ws(ctypes.byref(p), ws.data_ptr(), nbytes, _stream(dev)))
         else:
             _lib.check(L.mykfa_fwd(ctypes.byref(p), _stream(dev)))
     return out, lse

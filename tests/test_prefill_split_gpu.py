@@ -1,0 +1,49 @@
+"""The forward with split keys (few query blocks, long caches) against the oracle: sequences of
+no key, of one part and of many, partial tiles, windows, every head_dim, a negative scale, and
+the smallest and largest query counts that take it."""
+
+import pytest
+import torch
+
+from _util import assert_close, assert_lse
+from myk_llm_amd import flash_attn_func, flash_attn_with_kvcache
+from oracle.attention import kvcache_reference, reference_with_lse
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nq, heads, kv_heads, d, lens, window, scale, dtype", [
+    (17, 16, 4, 128, [0, 1, 1400], (-1, -1), None, torch.bfloat16),
+    (33, 8, 2, 64, [255, 256, 257, 2015], (-1, -1), None, torch.float16),
+    (130, 4, 4, 64, [2040, 63], (-1, -1), None, torch.bfloat16),
+    (64, 6, 2, 128, [1900], (1500, 0), None, torch.bfloat16),
+    (40, 3, 1, 32, [2000, 0], (-1, -1), -0.2, torch.bfloat16),
+    (100, 5, 5, 16, [1500], (-1, 7), None, torch.float16),
+    (31, 8, 1, 256, [1000, 30], (-1, -1), None, torch.bfloat16),
+])
+def test_split_keys_match_oracle(nq, heads, kv_heads, d, lens, window, scale, dtype):
+    print(f"split keys nq={nq} H={heads}/{kv_heads} D={d} lens={lens}", flush=True)
+    g = torch.Generator().manual_seed(nq)
+    b, cap = len(lens), 2200
+    mk = lambda *s: torch.randn(*s, generator=g).to(dtype)  # noqa: E731
+    q, kc, vc, kn, vn = mk(b, nq, heads, d), mk(b, cap, kv_heads, d), mk(b, cap, kv_heads, d), mk(b, nq, kv_heads, d), mk(b, nq, kv_heads, d)
+    cl = torch.tensor(lens, dtype=torch.int32)
+    causal = window[1] <= 0
+    exp, exp_lse, _, _ = kvcache_reference(q.float(), kc.float(), vc.float(), kn.float(), vn.float(), cl, causal,
+                                           window, scale)
+    out, lse = flash_attn_with_kvcache(q.cuda(), kc.cuda(), vc.cuda(), kn.cuda(), vn.cuda(), cache_seqlens=cl.cuda(),
+                                       causal=causal, window_size=window, softmax_scale=scale, return_softmax_lse=True)
+    assert_close(out, exp)
+    assert_lse(lse, exp_lse)
+
+
+@pytest.mark.parametrize("sq, sk, heads", [(1024, 1024, 16), (1025, 1025, 16), (700, 1111, 8)])
+def test_dense_batches_around_the_rule(sq, sk, heads):
+    """One causal sequence on both sides of the most rows that are split, and Lq != Lk."""
+    g = torch.Generator().manual_seed(sq)
+    mk = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)  # noqa: E731
+    q, k, v = mk(1, sq, heads, 64), mk(1, sk, heads // 4, 64), mk(1, sk, heads // 4, 64)
+    out, lse = flash_attn_func(q.cuda(), k.cuda(), v.cuda(), causal=True, return_softmax_lse=True)
+    exp, exp_lse = reference_with_lse(q, k, v, True, (-1, -1))
+    assert_close(out, exp)
+    assert_lse(lse, exp_lse)

@@ -45,6 +45,7 @@ extern "C" {
 /* Element types of q/k/v/o (reference accepts bf16 and fp16: flash_attn.py:340-341). */
 #define MYKFA_BF16 0
 #define MYKFA_FP16 1
+#define MYKFA_FP32 2 /* results of mykfa_gemm only */
 
 /* hipStream_t, without requiring the HIP headers in FFI users. NULL = default stream. */
 typedef struct ihipStream_t* mykfa_stream_t;
@@ -294,6 +295,50 @@ typedef struct mykfa_syrk_params {
     int32_t dtype; /* MYKFA_BF16 */
 } mykfa_syrk_params;
 
+/*
+ * Batched bf16 matrix products with fp32 accumulation: the products of fused_linear_cross_entropy
+ * (ops/fused_ce.py:70-108) and of Muon's Newton-Schulz step (ops/muon.py:218-268).
+ *   bf16 C: C[b] = alpha * A[b] B[b] + beta * Add[b]     (Add NULL: none; one rounding, at the store)
+ *   fp32 C: C[b] = A[b] B[b] + beta * C[b]
+ * A is (m, k), or (k, m) with a_transposed; B is (k, n), or (n, k) with b_transposed; rows with a
+ * contiguous last dimension, 16-byte aligned, strides multiples of 8 elements (C fp32: 4). A row is
+ * read up to the next multiple of 8 elements: what lies past k must be finite where the other
+ * operand has k rows, and zero where both have k columns; the pads of C's rows up to a multiple of
+ * 8 columns are stored too (zeros for bf16 without Add).
+ * symmetric: B = A^T (b ignored, n = m), Add symmetric; only the tiles on and below the diagonal
+ * are computed and mirrored, no pad of C is stored, and C and Add need only the alignment of
+ * mykfa_syrk.
+ * Supported: bf16 C with a_transposed = 0; fp32 C with a_transposed = 1 and b_transposed = 0.
+ */
+typedef struct mykfa_gemm_params {
+    const void* a;
+    const void* b;
+    const void* add;
+    void* c;
+    int64_t a_batch_stride, a_row_stride;
+    int64_t b_batch_stride, b_row_stride;
+    int64_t add_batch_stride, add_row_stride;
+    int64_t c_batch_stride, c_row_stride;
+    int32_t batch, m, n, k;
+    int32_t a_transposed, b_transposed, symmetric;
+    float alpha, beta;
+    int32_t c_dtype; /* MYKFA_BF16 / MYKFA_FP32 */
+} mykfa_gemm_params;
+
+/*
+ * Newton-Schulz iteration on a batch of matrices (batched_newton_schulz_orthogonalize,
+ * ops/muon.py:218-268): x (batch, rows, cols) bf16, contiguous, divided by its Frobenius norm (at
+ * least eps) unless `normalized`, iterated `steps` times with the quintic's coefficients a, b, c
+ * (on its transpose with `transposed`), into out (batch, rows, cols), contiguous.
+ */
+typedef struct mykfa_newton_schulz_params {
+    const void* x;
+    void* out;
+    int32_t batch, rows, cols;
+    int32_t transposed, normalized, steps;
+    float a, b, c, eps;
+} mykfa_newton_schulz_params;
+
 /* ---- version / errors ------------------------------------------------------------- */
 int mykfa_abi_version(void);
 const char* mykfa_version(void);
@@ -436,6 +481,20 @@ int mykfa_validate_syrk(const mykfa_syrk_params* p);
 /* out = alpha x x^T + beta bias over lower-triangular tiles (replaces _batched_syrk_kernel,
  * ops/muon.py:28-104, and its launcher batched_syrk, :107-143). */
 int mykfa_syrk(const mykfa_syrk_params* p, mykfa_stream_t stream);
+
+/* ---- Muon: Newton-Schulz ---------------------------------------------------------------- */
+size_t mykfa_sizeof_newton_schulz_params(void);
+int mykfa_validate_newton_schulz(const mykfa_newton_schulz_params* p);
+size_t mykfa_newton_schulz_workspace_size(const mykfa_newton_schulz_params* p);
+int mykfa_newton_schulz(const mykfa_newton_schulz_params* p, void* workspace, size_t workspace_bytes,
+                        mykfa_stream_t stream);
+
+/* ---- matrix products ------------------------------------------------------------------ */
+size_t mykfa_sizeof_gemm_params(void);
+int mykfa_validate_gemm(const mykfa_gemm_params* p);
+/* Workspace of products with few output tiles and a long k, which run in k splits (0: none). */
+size_t mykfa_gemm_workspace_size(const mykfa_gemm_params* p);
+int mykfa_gemm(const mykfa_gemm_params* p, void* workspace, size_t workspace_bytes, mykfa_stream_t stream);
 
 #ifdef __cplusplus
 }

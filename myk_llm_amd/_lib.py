@@ -24,6 +24,7 @@ DECODE_SCRATCH_BYTES = 16 << 20  # MYKFA_DECODE_SCRATCH_BYTES
 
 DTYPE_BF16 = 0
 DTYPE_FP16 = 1
+DTYPE_FP32 = 2  # results of mykfa_gemm only
 UNBOUNDED = 1 << 30
 
 _i64, _i32, _f32, _ptr = ctypes.c_int64, ctypes.c_int32, ctypes.c_float, ctypes.c_void_p
@@ -133,6 +134,25 @@ class SyrkParams(ctypes.Structure):
     ]
 
 
+class GemmParams(ctypes.Structure):
+    _fields_ = [
+        ("a", _ptr), ("b", _ptr), ("add", _ptr), ("c", _ptr),
+        ("a_batch_stride", _i64), ("a_row_stride", _i64), ("b_batch_stride", _i64), ("b_row_stride", _i64),
+        ("add_batch_stride", _i64), ("add_row_stride", _i64), ("c_batch_stride", _i64), ("c_row_stride", _i64),
+        ("batch", _i32), ("m", _i32), ("n", _i32), ("k", _i32),
+        ("a_transposed", _i32), ("b_transposed", _i32), ("symmetric", _i32),
+        ("alpha", _f32), ("beta", _f32), ("c_dtype", _i32),
+    ]
+
+
+class NewtonSchulzParams(ctypes.Structure):
+    _fields_ = [
+        ("x", _ptr), ("out", _ptr), ("batch", _i32), ("rows", _i32), ("cols", _i32),
+        ("transposed", _i32), ("normalized", _i32), ("steps", _i32),
+        ("a", _f32), ("b", _f32), ("c", _f32), ("eps", _f32),
+    ]
+
+
 # Every symbol include/mykfa.h declares, with (restype, argtypes).
 SIGNATURES = {
     "mykfa_abi_version": (ctypes.c_int, []),
@@ -181,6 +201,14 @@ SIGNATURES = {
     "mykfa_sizeof_syrk_params": (ctypes.c_size_t, []),
     "mykfa_validate_syrk": (ctypes.c_int, [ctypes.POINTER(SyrkParams)]),
     "mykfa_syrk": (ctypes.c_int, [ctypes.POINTER(SyrkParams), _ptr]),
+    "mykfa_sizeof_newton_schulz_params": (ctypes.c_size_t, []),
+    "mykfa_validate_newton_schulz": (ctypes.c_int, [ctypes.POINTER(NewtonSchulzParams)]),
+    "mykfa_newton_schulz_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(NewtonSchulzParams)]),
+    "mykfa_newton_schulz": (ctypes.c_int, [ctypes.POINTER(NewtonSchulzParams), _ptr, ctypes.c_size_t, _ptr]),
+    "mykfa_sizeof_gemm_params": (ctypes.c_size_t, []),
+    "mykfa_validate_gemm": (ctypes.c_int, [ctypes.POINTER(GemmParams)]),
+    "mykfa_gemm_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(GemmParams)]),
+    "mykfa_gemm": (ctypes.c_int, [ctypes.POINTER(GemmParams), _ptr, ctypes.c_size_t, _ptr]),
 }
 
 _STRUCT_SIZES = {
@@ -193,6 +221,8 @@ _STRUCT_SIZES = {
     "mykfa_sizeof_gate_params": GateParams,
     "mykfa_sizeof_ce_params": CeParams,
     "mykfa_sizeof_syrk_params": SyrkParams,
+    "mykfa_sizeof_gemm_params": GemmParams,
+    "mykfa_sizeof_newton_schulz_params": NewtonSchulzParams,
 }
 
 def _flat_layout(struct_type, base: int = 0, out=None):
@@ -228,6 +258,7 @@ def _packer(struct_type) -> struct.Struct:
 FWD_PACK = _packer(FwdParams)
 BWD_PACK = _packer(BwdParams)
 DECODE_PACK = _packer(DecodeParams)
+GEMM_PACK = _packer(GemmParams)
 
 
 _lib: ctypes.CDLL | None = None

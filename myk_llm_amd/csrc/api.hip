@@ -313,6 +313,80 @@ int check_syrk(const mykfa_syrk_params* p) {
     return MYKFA_OK;
 }
 
+// One operand or result of a product: rows of a contiguous last dimension, `align` elements of
+// alignment, and a tile of `tile` rows within a buffer descriptor's 2 GiB.
+int check_matrix(const void* ptr, int64_t bs, int64_t rs, int64_t cols, int align, int tile, const char* name) {
+    if (ptr == nullptr || !aligned16(ptr)) return fail(MYKFA_ERR_INVALID, "%s must be non-NULL and 16-byte aligned", name);
+    if (bs < 0 || bs % align != 0 || rs % align != 0 || rs < (cols + 7) / 8 * 8)
+        return fail(MYKFA_ERR_INVALID,
+                    "%s strides (%lld, %lld) must be multiples of %d elements, rows at least their %lld columns rounded up to 8",
+                    name, (long long)bs, (long long)rs, align, (long long)cols);
+    if (((tile - 1) * rs + cols + 8) * 2 > 0x7fffffffLL)
+        return fail(MYKFA_ERR_UNSUPPORTED, "%d rows of %s at row stride %lld span more than 2 GiB", tile, name, (long long)rs);
+    return MYKFA_OK;
+}
+
+// The products of ops/fused_ce.py:70-108 and ops/muon.py:218-268.
+int check_gemm(const mykfa_gemm_params* p) {
+    if (p == nullptr) return fail(MYKFA_ERR_INVALID, "params is NULL");
+    if (p->batch < 0 || p->m < 0 || p->n < 0 || p->k < 0)
+        return fail(MYKFA_ERR_INVALID, "negative shape (batch %d, m %d, n %d, k %d)", p->batch, p->m, p->n, p->k);
+    if (p->c_dtype != MYKFA_BF16 && p->c_dtype != MYKFA_FP32)
+        return fail(MYKFA_ERR_UNSUPPORTED, "c_dtype must be bf16 or fp32; got code %d", p->c_dtype);
+    if (p->c_dtype == MYKFA_FP32 ? !p->a_transposed || p->b_transposed || p->symmetric || p->add != nullptr
+                                 : p->a_transposed != 0)
+        return fail(MYKFA_ERR_UNSUPPORTED, "no kernel for a_transposed %d, b_transposed %d, symmetric %d with c_dtype %d",
+                    p->a_transposed, p->b_transposed, p->symmetric, p->c_dtype);
+    if (!(p->alpha == p->alpha) || !(p->beta == p->beta)) return fail(MYKFA_ERR_INVALID, "alpha or beta is NaN");
+    const long long t = ((long long)p->m + 63) / 64 * (((long long)p->n + 63) / 64);
+    if (t > (1ll << 30) || t * p->batch > (1ll << 30))
+        return fail(MYKFA_ERR_UNSUPPORTED, "batch %d of %d x %d exceeds the grid limit", p->batch, p->m, p->n);
+    if (p->symmetric && p->n != p->m) return fail(MYKFA_ERR_INVALID, "symmetric needs n (%d) = m (%d)", p->n, p->m);
+    if (p->symmetric && p->k % 8 != 0) return fail(MYKFA_ERR_UNSUPPORTED, "symmetric needs k (%d) a multiple of 8", p->k);
+    if (p->batch == 0 || p->m == 0 || p->n == 0) return MYKFA_OK;
+    int rc;
+    if (p->symmetric) {
+        if (p->c == nullptr || (reinterpret_cast<uintptr_t>(p->c) & 7) != 0)
+            return fail(MYKFA_ERR_INVALID, "c must be non-NULL and 8-byte aligned");
+        if (p->c_row_stride < p->m || (p->c_row_stride & 3) != 0 || p->c_batch_stride < 0)
+            return fail(MYKFA_ERR_INVALID, "c row stride %lld must be >= m and a multiple of 4", (long long)p->c_row_stride);
+        if (p->add != nullptr && ((reinterpret_cast<uintptr_t>(p->add) & 1) != 0 || p->add_row_stride < 0 ||
+                                  p->add_batch_stride < 0))
+            return fail(MYKFA_ERR_INVALID, "add must be 2-byte aligned with non-negative strides");
+    } else {
+        if ((rc = check_matrix(p->c, p->c_batch_stride, p->c_row_stride, p->n, p->c_dtype == MYKFA_FP32 ? 4 : 8, 1, "c"))) return rc;
+        if (p->add != nullptr &&
+            (rc = check_matrix(p->add, p->add_batch_stride, p->add_row_stride, p->n, 8, 1, "add"))) return rc;
+    }
+    if (p->k == 0) return MYKFA_OK;
+    if ((rc = check_matrix(p->a, p->a_batch_stride, p->a_row_stride, p->a_transposed ? p->m : p->k, 8, p->a_transposed ? 64 : p->symmetric ? 128 : 256, "a"))) return rc;
+    if (!p->symmetric &&
+        (rc = check_matrix(p->b, p->b_batch_stride, p->b_row_stride, p->b_transposed ? p->k : p->n, 8, p->b_transposed ? 256 : 64, "b"))) return rc;
+    return MYKFA_OK;
+}
+
+// ops/muon.py:218-268.
+int check_newton_schulz(const mykfa_newton_schulz_params* p) {
+    if (p == nullptr) return fail(MYKFA_ERR_INVALID, "params is NULL");
+    if (p->batch < 0 || p->rows < 0 || p->cols < 0 || p->steps < 0)
+        return fail(MYKFA_ERR_INVALID, "negative shape (batch %d, %d x %d) or steps (%d)", p->batch, p->rows, p->cols, p->steps);
+    if (!(p->a == p->a) || !(p->b == p->b) || !(p->c == p->c) || !(p->eps == p->eps))
+        return fail(MYKFA_ERR_INVALID, "a coefficient or eps is NaN");
+    if (p->batch > 65535) return fail(MYKFA_ERR_UNSUPPORTED, "batch %d exceeds the grid limit 65535", p->batch);
+    if (p->rows >= (1 << 23) || p->cols >= (1 << 23))  // 128 rows within a buffer descriptor's 2 GiB
+        return fail(MYKFA_ERR_UNSUPPORTED, "%d x %d: a dimension of 2^23 or more", p->rows, p->cols);
+    if ((long long)p->batch * p->rows * p->cols == 0) return MYKFA_OK;
+    {
+        const long long m = p->transposed ? p->cols : p->rows, k = p->transposed ? p->rows : p->cols;
+        if ((m + 63) / 64 * (((m > k ? m : k) + 63) / 64) * p->batch > (1ll << 30))
+            return fail(MYKFA_ERR_UNSUPPORTED, "batch %d of %d x %d exceeds the grid limit", p->batch, p->rows, p->cols);
+    }
+    if (p->x == nullptr || p->out == nullptr || (reinterpret_cast<uintptr_t>(p->x) & 1) != 0 ||
+        (reinterpret_cast<uintptr_t>(p->out) & 1) != 0)
+        return fail(MYKFA_ERR_INVALID, "x and out must be non-NULL and 2-byte aligned");
+    return MYKFA_OK;
+}
+
 hipStream_t as_stream(mykfa_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 int choose_splits(const mykfa_decode_params* p) {
@@ -597,6 +671,54 @@ int mykfa_syrk(const mykfa_syrk_params* p, mykfa_stream_t stream) {
     if (rc) return rc;
     if (p->batch == 0 || p->m == 0) return ok();
     return launched(mykfa::launch_syrk(*p, as_stream(stream)), "mykfa_syrk");
+}
+
+size_t mykfa_sizeof_newton_schulz_params(void) { return sizeof(mykfa_newton_schulz_params); }
+
+int mykfa_validate_newton_schulz(const mykfa_newton_schulz_params* p) {
+    int rc = check_newton_schulz(p);
+    return rc ? rc : ok();
+}
+
+size_t mykfa_newton_schulz_workspace_size(const mykfa_newton_schulz_params* p) {
+    if (check_newton_schulz(p)) return 0;
+    return mykfa::newton_schulz_bytes(*p);
+}
+
+int mykfa_newton_schulz(const mykfa_newton_schulz_params* p, void* workspace, size_t workspace_bytes,
+                        mykfa_stream_t stream) {
+    int rc = check_newton_schulz(p);
+    if (rc) return rc;
+    if ((long long)p->batch * p->rows * p->cols == 0) return ok();
+    const size_t need = mykfa::newton_schulz_bytes(*p);
+    if (workspace == nullptr || workspace_bytes < need)
+        return fail(MYKFA_ERR_WORKSPACE, "mykfa_newton_schulz needs %zu bytes of workspace; got %zu", need, workspace_bytes);
+    if ((reinterpret_cast<uintptr_t>(workspace) & 255) != 0)
+        return fail(MYKFA_ERR_INVALID, "mykfa_newton_schulz: workspace must be 256-byte aligned");
+    return launched(mykfa::launch_newton_schulz(*p, workspace, as_stream(stream)), "mykfa_newton_schulz");
+}
+
+size_t mykfa_sizeof_gemm_params(void) { return sizeof(mykfa_gemm_params); }
+
+int mykfa_validate_gemm(const mykfa_gemm_params* p) {
+    int rc = check_gemm(p);
+    return rc ? rc : ok();
+}
+
+size_t mykfa_gemm_workspace_size(const mykfa_gemm_params* p) {
+    if (check_gemm(p)) return 0;
+    return mykfa::gemm_workspace_bytes(*p);
+}
+
+int mykfa_gemm(const mykfa_gemm_params* p, void* workspace, size_t workspace_bytes, mykfa_stream_t stream) {
+    int rc = check_gemm(p);
+    if (rc) return rc;
+    if (p->batch == 0 || p->m == 0 || p->n == 0) return ok();
+    const size_t need = mykfa::gemm_workspace_bytes(*p);
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
+        return fail(MYKFA_ERR_WORKSPACE, "mykfa_gemm needs %zu bytes of workspace; got %zu", need, workspace_bytes);
+    if (need > 0 && !aligned16(workspace)) return fail(MYKFA_ERR_INVALID, "mykfa_gemm: workspace must be 16-byte aligned");
+    return launched(mykfa::launch_gemm(*p, workspace, as_stream(stream)), "mykfa_gemm");
 }
 
 size_t mykfa_sizeof_ce_params(void) { return sizeof(mykfa_ce_params); }

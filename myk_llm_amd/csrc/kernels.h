@@ -51,7 +51,11 @@ hipError_t launch_gate(const mykfa_gate_params& p, bool backward, hipStream_t st
 // Cross-entropy rows of the fused linear + cross-entropy (fused_ce.hip).
 hipError_t launch_ce_rows(const mykfa_ce_params& p, hipStream_t stream);
 
-// Batched SYRK of Muon's Newton-Schulz iteration (syrk.hip).
+// Batched matrix products and Muon's SYRK (gemm.hip); its Newton-Schulz iteration (muon.hip).
+size_t gemm_workspace_bytes(const mykfa_gemm_params& p);
+hipError_t launch_gemm(const mykfa_gemm_params& p, void* ws, hipStream_t stream);
+size_t newton_schulz_bytes(const mykfa_newton_schulz_params& p);
+hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, hipStream_t stream);
 hipError_t launch_syrk(const mykfa_syrk_params& p, hipStream_t stream);
 
 }  // namespace mykfa

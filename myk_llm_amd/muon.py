@@ -8,15 +8,13 @@ myk-llm's src/myk_llm/ops/muon.py (exported by ops/__init__.py), same names and 
         the quintic Newton-Schulz iteration on a batch of matrices (ops/muon.py:218-268):
         per step G = X X^T and G2 = b G + c G G through batched_syrk, X' = a X + G2 X
 
-The SYRK runs in the hand-written gfx950 kernel of libmykfa.so (csrc/syrk.hip) through its C
-ABI; the third product of each step (a general matrix product) is a library GEMM
-(torch.baddbmm = hipBLASLt), as in the reference (cuBLAS baddbmm).
+Every product runs in the hand-written gfx950 kernels of libmykfa.so (csrc/gemm.hip); the whole
+iteration is one call of its C ABI (csrc/muon.hip: norms, scaled copy, three products a step).
 
 Differences from the reference's layout handling: the kernel reads k-contiguous rows whose
-length is a multiple of 64, so transposed or strided x and unaligned k are copied once
-(zero-padded) before the call; the Newton-Schulz driver transposes tall matrices with one
-contiguous copy instead of iterating on transposed views (batched bf16 products on transposed
-views are avoided on this platform).
+length is a multiple of 8, so transposed or strided x and unaligned k are copied once
+(zero-padded) before the call; the Newton-Schulz driver iterates tall matrices on a transposed
+copy instead of transposed views.
 """
 
 from __future__ import annotations
@@ -29,17 +27,16 @@ from torch import Tensor
 
 from . import _lib
 from .flash_attn import _DeviceGuard, _same_device, _stream
+from .gemm import gemm, usable
 
 NS_COEFFICIENTS = (3.4445, -4.7750, 2.0315)  # ops/muon.py:25
 
 
 def _kernel_x(x: Tensor) -> Tensor:
-    """x as (B, M, Kp) bf16 rows with Kp a multiple of 64, 16-byte aligned, row stride 8k."""
+    """x as (B, M, Kp) bf16 rows with Kp a multiple of 8, 16-byte aligned, row stride 8k."""
     b, m, k = x.shape
-    kp = (k + 63) // 64 * 64
-    ok = (x.stride(2) == 1 and kp == k and x.data_ptr() % 16 == 0 and x.stride(1) % 8 == 0
-          and x.stride(1) >= k and x.stride(0) >= 0)
-    if ok:
+    kp = (k + 7) // 8 * 8
+    if kp == k and usable(x):
         return x
     xp = torch.zeros((b, m, kp), dtype=torch.bfloat16, device=x.device)
     xp[..., :k] = x
@@ -72,18 +69,9 @@ def batched_syrk(x: Tensor, bias: Optional[Tensor] = None, alpha: float = 1.0, b
         o = torch.empty((B, M, (M + 3) // 4 * 4), device=x.device, dtype=torch.bfloat16)[:, :, :M]
     if bias is not None and (bias.stride(2) != 1 or bias.data_ptr() % 2):
         bias = bias.contiguous()
-    p = _lib.SyrkParams()
-    p.x, p.out = xk.data_ptr(), o.data_ptr()
-    p.x_batch_stride, p.x_row_stride = xk.stride(0), xk.stride(1)
-    p.out_batch_stride, p.out_row_stride = o.stride(0), o.stride(1)
-    if bias is not None:
-        p.bias = bias.data_ptr()
-        p.bias_batch_stride, p.bias_row_stride = bias.stride(0), bias.stride(1)
-    p.batch, p.m, p.k = B, M, xk.shape[2]
-    p.alpha, p.beta = float(alpha), float(beta)
-    p.dtype = _lib.DTYPE_BF16
-    with _DeviceGuard(x.device):
-        _lib.check(_lib.lib().mykfa_syrk(ctypes.byref(p), _stream(x.device)))
+    if B > 0 and M > 0:
+        with _DeviceGuard(x.device):
+            gemm(xk, None, o, M, M, xk.shape[2], symmetric=True, add=bias, alpha=float(alpha), beta=float(beta))
     if o is not out:
         out.copy_(o)
     return out
@@ -120,17 +108,19 @@ def batched_newton_schulz_orthogonalize(packed: Tensor, steps: int, transposed: 
     if norm_sq is not None:
         inv = 1.0 / torch.clamp(norm_sq.reshape(B, 1, 1).float().sqrt(), min=eps)
         packed.copy_((packed.float() * inv).bfloat16())
-    else:
-        norm = _frobenius_norm(packed).reshape(B, 1, 1).clamp_(min=eps)
-        packed = (packed / norm).bfloat16()
-    x = packed.transpose(-2, -1).contiguous() if transposed else packed
-    M = x.size(1)
-    gram = torch.empty((B, M, M), device=x.device, dtype=torch.bfloat16)
-    gram2 = torch.empty((B, M, M), device=x.device, dtype=torch.bfloat16)
-    x_next = torch.empty_like(x)
-    for _ in range(steps):
-        batched_syrk(x, out=gram)
-        batched_syrk(gram, bias=gram, alpha=c, beta=b, out=gram2)
-        torch.baddbmm(x, gram2, x, beta=a, alpha=1.0, out=x_next)
-        x, x_next = x_next, x
-    return x.transpose(-2, -1).contiguous() if transposed else x
+    if steps <= 0 or packed.numel() == 0:
+        if norm_sq is None:
+            packed = (packed / _frobenius_norm(packed).reshape(B, 1, 1).clamp_(min=eps)).bfloat16()
+        return packed
+    if not packed.is_cuda:
+        raise RuntimeError("batched Newton-Schulz is CUDA-only: packed must be a GPU (HIP) tensor")
+    if torch.is_grad_enabled() and packed.requires_grad:
+        raise RuntimeError("batched Newton-Schulz has no gradient: packed must not require one")
+    out = torch.empty_like(packed)
+    p = _lib.NewtonSchulzParams(packed.data_ptr(), out.data_ptr(), B, rows, cols, bool(transposed),
+                                norm_sq is not None, steps, a, b, c, eps)
+    L = _lib.lib()
+    with _DeviceGuard(packed.device):
+        ws = torch.empty(L.mykfa_newton_schulz_workspace_size(ctypes.byref(p)), dtype=torch.uint8, device=packed.device)
+        _lib.check(L.mykfa_newton_schulz(ctypes.byref(p), ws.data_ptr(), ws.numel(), _stream(packed.device)))
+    return out

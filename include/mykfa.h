@@ -45,7 +45,7 @@ extern "C" {
 /* Element types of q/k/v/o (reference accepts bf16 and fp16: flash_attn.py:340-341). */
 #define MYKFA_BF16 0
 #define MYKFA_FP16 1
-#define MYKFA_FP32 2 /* results of mykfa_gemm only */
+#define MYKFA_FP32 2 /* mykfa_gemm's results, mykfa_scale */
 
 /* hipStream_t, without requiring the HIP headers in FFI users. NULL = default stream. */
 typedef struct ihipStream_t* mykfa_stream_t;
@@ -339,6 +339,28 @@ typedef struct mykfa_newton_schulz_params {
     float a, b, c, eps;
 } mykfa_newton_schulz_params;
 
+/* loss = (ce_sum + z_coef * z_sum) * scale with ce_sum = sum of ce and z_sum = sum of lse^2 over
+ * `rows` tokens (ops/fused_ce.py:111-132); one workgroup, meant for up to some 10^5 tokens. */
+typedef struct mykfa_ce_loss_params {
+    const float* ce;
+    const float* lse;
+    float* loss;
+    float* ce_sum;
+    float* z_sum;
+    int64_t rows;
+    float scale, z_coef;
+} mykfa_ce_loss_params;
+
+/* dst[i] = src[i] * *factor, the product rounded to the source's type and cast to the
+ * destination's: the stored gradients times the loss's (ops/fused_ce.py:98-108). */
+typedef struct mykfa_scale_params {
+    const void* src; /* bf16 or fp32, contiguous, 16-byte aligned */
+    void* dst;       /* bf16, fp16 or fp32, likewise */
+    const float* factor;
+    int64_t n;
+    int32_t src_dtype, dst_dtype;
+} mykfa_scale_params;
+
 /* ---- version / errors ------------------------------------------------------------- */
 int mykfa_abi_version(void);
 const char* mykfa_version(void);
@@ -481,6 +503,11 @@ int mykfa_validate_syrk(const mykfa_syrk_params* p);
 /* out = alpha x x^T + beta bias over lower-triangular tiles (replaces _batched_syrk_kernel,
  * ops/muon.py:28-104, and its launcher batched_syrk, :107-143). */
 int mykfa_syrk(const mykfa_syrk_params* p, mykfa_stream_t stream);
+
+size_t mykfa_sizeof_ce_loss_params(void);
+int mykfa_ce_loss(const mykfa_ce_loss_params* p, mykfa_stream_t stream);
+size_t mykfa_sizeof_scale_params(void);
+int mykfa_scale(const mykfa_scale_params* p, mykfa_stream_t stream);
 
 /* ---- Muon: Newton-Schulz ---------------------------------------------------------------- */
 size_t mykfa_sizeof_newton_schulz_params(void);

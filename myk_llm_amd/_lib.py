@@ -145,6 +145,19 @@ class GemmParams(ctypes.Structure):
     ]
 
 
+class CeLossParams(ctypes.Structure):
+    _fields_ = [
+        ("ce", _ptr), ("lse", _ptr), ("loss", _ptr), ("ce_sum", _ptr), ("z_sum", _ptr),
+        ("rows", _i64), ("scale", _f32), ("z_coef", _f32),
+    ]
+
+
+class ScaleParams(ctypes.Structure):
+    _fields_ = [
+        ("src", _ptr), ("dst", _ptr), ("factor", _ptr), ("n", _i64), ("src_dtype", _i32), ("dst_dtype", _i32),
+    ]
+
+
 class NewtonSchulzParams(ctypes.Structure):
     _fields_ = [
         ("x", _ptr), ("out", _ptr), ("batch", _i32), ("rows", _i32), ("cols", _i32),
@@ -201,6 +214,10 @@ SIGNATURES = {
     "mykfa_sizeof_syrk_params": (ctypes.c_size_t, []),
     "mykfa_validate_syrk": (ctypes.c_int, [ctypes.POINTER(SyrkParams)]),
     "mykfa_syrk": (ctypes.c_int, [ctypes.POINTER(SyrkParams), _ptr]),
+    "mykfa_sizeof_ce_loss_params": (ctypes.c_size_t, []),
+    "mykfa_ce_loss": (ctypes.c_int, [ctypes.POINTER(CeLossParams), _ptr]),
+    "mykfa_sizeof_scale_params": (ctypes.c_size_t, []),
+    "mykfa_scale": (ctypes.c_int, [ctypes.POINTER(ScaleParams), _ptr]),
     "mykfa_sizeof_newton_schulz_params": (ctypes.c_size_t, []),
     "mykfa_validate_newton_schulz": (ctypes.c_int, [ctypes.POINTER(NewtonSchulzParams)]),
     "mykfa_newton_schulz_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(NewtonSchulzParams)]),
@@ -223,6 +240,8 @@ _STRUCT_SIZES = {
     "mykfa_sizeof_syrk_params": SyrkParams,
     "mykfa_sizeof_gemm_params": GemmParams,
     "mykfa_sizeof_newton_schulz_params": NewtonSchulzParams,
+    "mykfa_sizeof_ce_loss_params": CeLossParams,
+    "mykfa_sizeof_scale_params": ScaleParams,
 }
 
 def _flat_layout(struct_type, base: int = 0, out=None):

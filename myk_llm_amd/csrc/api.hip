@@ -673,6 +673,31 @@ int mykfa_syrk(const mykfa_syrk_params* p, mykfa_stream_t stream) {
     return launched(mykfa::launch_syrk(*p, as_stream(stream)), "mykfa_syrk");
 }
 
+size_t mykfa_sizeof_ce_loss_params(void) { return sizeof(mykfa_ce_loss_params); }
+
+int mykfa_ce_loss(const mykfa_ce_loss_params* p, mykfa_stream_t stream) {
+    if (p == nullptr) return fail(MYKFA_ERR_INVALID, "params is NULL");
+    if (p->rows < 0) return fail(MYKFA_ERR_INVALID, "negative rows (%lld)", (long long)p->rows);
+    if (p->loss == nullptr || p->ce_sum == nullptr || p->z_sum == nullptr ||
+        (p->rows > 0 && (p->ce == nullptr || p->lse == nullptr)))
+        return fail(MYKFA_ERR_INVALID, "ce, lse, loss, ce_sum and z_sum must be non-NULL");
+    return launched(mykfa::launch_ce_loss(*p, as_stream(stream)), "mykfa_ce_loss");
+}
+
+size_t mykfa_sizeof_scale_params(void) { return sizeof(mykfa_scale_params); }
+
+int mykfa_scale(const mykfa_scale_params* p, mykfa_stream_t stream) {
+    if (p == nullptr) return fail(MYKFA_ERR_INVALID, "params is NULL");
+    if (p->n < 0) return fail(MYKFA_ERR_INVALID, "negative n (%lld)", (long long)p->n);
+    if ((p->src_dtype != MYKFA_BF16 && p->src_dtype != MYKFA_FP32) || p->dst_dtype < MYKFA_BF16 || p->dst_dtype > MYKFA_FP32)
+        return fail(MYKFA_ERR_UNSUPPORTED, "no scaling from dtype code %d to %d", p->src_dtype, p->dst_dtype);
+    if (p->n == 0) return ok();
+    if (p->src == nullptr || p->dst == nullptr || p->factor == nullptr || !aligned16(p->src) || !aligned16(p->dst) ||
+        (reinterpret_cast<uintptr_t>(p->factor) & 3) != 0)
+        return fail(MYKFA_ERR_INVALID, "src and dst must be 16-byte aligned, factor 4-byte, all non-NULL");
+    return launched(mykfa::launch_scale(*p, as_stream(stream)), "mykfa_scale");
+}
+
 size_t mykfa_sizeof_newton_schulz_params(void) { return sizeof(mykfa_newton_schulz_params); }
 
 int mykfa_validate_newton_schulz(const mykfa_newton_schulz_params* p) {

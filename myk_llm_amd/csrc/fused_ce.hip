@@ -6,12 +6,16 @@
 // ce_rows_resident_kernel: rows of up to 512 * VPT columns (65536 at VPT = 128, the
 //   reference's 64K vocabulary) are held in registers, so each logit is read from HBM once and
 //   written once (the reference streams the row twice: one pass for the statistics, one for the
-//   gradient). 16-byte accesses: the vocabulary and the row stride are multiples of 8.
+//   gradient). 16-byte accesses: the row stride is a multiple of 8; the columns of a vocabulary
+//   past its last multiple of 8 (TAIL) are the business of one lane, element by element (1531
+//   rows of 32003 columns: 139 us through the streaming kernel before, 22 now).
 // ce_rows_stream_kernel: any other shape (larger vocabularies, unaligned rows): two passes
 //   over the row, an online max/sum per lane first.
 // Block reductions are fixed-order (lane shuffles, then the 8 waves in order through LDS):
 // results are bitwise repeatable.
 #include <math.h>
+
+#include <type_traits>
 
 #include "common.h"
 #include "kernels.h"
@@ -79,7 +83,11 @@ template <typename T>
 __device__ inline void zero_row(uint16_t* base, int vocab, bool vec) {
     if (vec) {
         const s16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (int c = threadIdx.x * 8; c < vocab; c += kCeThreads * 8) st16(base + c, z);
+        for (int c = threadIdx.x * 8; c < vocab; c += kCeThreads * 8) {
+            if (c + 8 <= vocab) st16(base + c, z);
+            else
+                for (int i = c; i < vocab; ++i) base[i] = 0;
+        }
     } else {
         for (int c = threadIdx.x; c < vocab; c += kCeThreads) base[c] = 0;
     }
@@ -122,7 +130,30 @@ __device__ inline uint32_t keep_code(float p) {  // p in [2^-63, 1] -> 16-bit co
 }
 __device__ inline float keep_value(uint32_t code) { return __uint_as_float((code << 13) + kKeepBias); }
 
-template <typename T, int VPT>
+// The 16-byte chunk of a row at column c: past the row's end (TAIL, its last chunk only) the
+// loaded columns are -inf, which adds nothing to the maximum or the sum, and none is stored.
+template <typename T, bool TAIL>
+__device__ inline s16x8 load_chunk(const uint16_t* base, int c, int vocab) {
+    if (!TAIL || c + 8 <= vocab) return ld16(base + c);
+    const short inf = T::code == MYKFA_BF16 ? (short)0xff80 : (short)0xfc00;
+    s16x8 v = {inf, inf, inf, inf, inf, inf, inf, inf};
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (c + i < vocab) v[i] = (short)base[c + i];
+    return v;
+}
+template <bool TAIL>
+__device__ inline void store_chunk(uint16_t* base, int c, int vocab, s16x8 v) {
+    if (!TAIL || c + 8 <= vocab) {
+        st16(base + c, v);
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        if (c + i < vocab) base[c + i] = (uint16_t)v[i];
+}
+
+template <typename T, int VPT, bool TAIL>
 __global__ __launch_bounds__(kCeThreads) void ce_rows_resident_kernel(mykfa_ce_params p) {
     constexpr int NC = VPT / 8;  // 16-byte chunks per lane
     constexpr bool kKeepP = T::code == MYKFA_BF16;
@@ -144,7 +175,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_resident_kernel(mykfa_ce_p
     for (int j = 0; j < NC; ++j) {
         const int c = (j * kCeThreads + threadIdx.x) * 8;
         if (c < p.vocab) {
-            v[j] = ld16(base + c);
+            v[j] = load_chunk<T, TAIL>(base, c, p.vocab);
 #pragma unroll
             for (int i = 0; i < 8; ++i) m = fmaxf(m, T::to_float((uint16_t)v[j][i]));
         }
@@ -202,7 +233,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_resident_kernel(mykfa_ce_p
                         ow[i] = T::pack2(keep_value(pw[i] & 0xffffu) * ratio, keep_value(pw[i] >> 16) * ratio);
                 }
                 const u32x4 o = {ow[0], ow[1], ow[2], ow[3]};
-                st16(base + c, __builtin_bit_cast(s16x8, o));
+                store_chunk<TAIL>(base, c, p.vocab, __builtin_bit_cast(s16x8, o));
             }
         }
         if (owner) {  // after this lane's store of the same 16 bytes
@@ -228,7 +259,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_resident_kernel(mykfa_ce_p
                 o[i] = (short)(w & 0xffff);
                 o[i + 1] = (short)(w >> 16);
             }
-            st16(base + c, o);
+            store_chunk<TAIL>(base, c, p.vocab, o);
         }
     }
 }
@@ -298,19 +329,128 @@ __global__ __launch_bounds__(kCeThreads) void ce_rows_stream_kernel(mykfa_ce_par
     }
 }
 
+template <typename T, bool TAIL>
+void ce_resident(const mykfa_ce_params& p, hipStream_t s) {
+    const dim3 grid((unsigned)p.rows), block(kCeThreads);
+    const int per_lane = (p.vocab + kCeThreads - 1) / kCeThreads;
+    if (per_lane <= 8) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 8, TAIL>), grid, block, 0, s, p);
+    else if (per_lane <= 16) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 16, TAIL>), grid, block, 0, s, p);
+    else if (per_lane <= 32) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 32, TAIL>), grid, block, 0, s, p);
+    else if (per_lane <= 64) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 64, TAIL>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((ce_rows_resident_kernel<T, 128, TAIL>), grid, block, 0, s, p);
+}
+
 template <typename T>
 hipError_t ce_dtype(const mykfa_ce_params& p, hipStream_t s) {
-    const dim3 grid((unsigned)p.rows), block(kCeThreads);
-    const bool vec = (p.vocab % 8) == 0 && (p.row_stride % 8) == 0 &&
-                     (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0;
-    const int per_lane = (p.vocab + kCeThreads - 1) / kCeThreads;
-    if (vec && per_lane <= 8) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 8>), grid, block, 0, s, p);
-    else if (vec && per_lane <= 16) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 16>), grid, block, 0, s, p);
-    else if (vec && per_lane <= 32) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 32>), grid, block, 0, s, p);
-    else if (vec && per_lane <= 64) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 64>), grid, block, 0, s, p);
-    else if (vec && per_lane <= 128) hipLaunchKernelGGL((ce_rows_resident_kernel<T, 128>), grid, block, 0, s, p);
-    else hipLaunchKernelGGL((ce_rows_stream_kernel<T>), grid, block, 0, s, p, vec ? 1 : 0);
+    const bool rows16 = (p.row_stride % 8) == 0 && (reinterpret_cast<uintptr_t>(p.logits) & 15) == 0;
+    if (rows16 && p.vocab <= kCeThreads * 128) {
+        if (p.vocab % 8 == 0) ce_resident<T, false>(p, s);
+        else ce_resident<T, true>(p, s);
+    } else {
+        const bool vec = rows16 && p.vocab % 8 == 0;
+        hipLaunchKernelGGL((ce_rows_stream_kernel<T>), dim3((unsigned)p.rows), dim3(kCeThreads), 0, s, p, vec ? 1 : 0);
+    }
     return hipGetLastError();
+}
+
+// ---- the loss and the scaled gradients ------------------------------------------------------
+
+// ce_sum, z_sum = sum lse^2 and loss = (ce_sum + z ce_sum) * scale over the tokens, by one workgroup
+// in double (order fixed): one launch of about 6 us where a sum, a dot and two scalar operations
+// were four.
+constexpr int kSumThreads = 1024;
+__global__ __launch_bounds__(kSumThreads) void ce_loss_kernel(mykfa_ce_loss_params p) {
+    __shared__ double red[2][kSumThreads / 64];
+    double ce = 0.0, z = 0.0;
+    for (int64_t i = threadIdx.x; i < p.rows; i += kSumThreads) {
+        const double l = p.lse[i];
+        ce += p.ce[i];
+        z += l * l;
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+        ce += __shfl_xor(ce, m);
+        z += __shfl_xor(z, m);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[0][threadIdx.x >> 6] = ce;
+        red[1][threadIdx.x >> 6] = z;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        ce = z = 0.0;
+        for (int i = 0; i < kSumThreads / 64; ++i) {
+            ce += red[0][i];
+            z += red[1][i];
+        }
+        *p.ce_sum = (float)ce;
+        *p.z_sum = (float)z;
+        *p.loss = ((float)ce + p.z_coef * (float)z) * p.scale;
+    }
+}
+
+// dst = src * *factor, rounded to the source's type and cast: what the backward does with the
+// stored gradients. One read and one write (torch's mul of a bf16 tensor by an fp32 scalar tensor
+// ran at 1.2 TB/s, and a second pass cast the product).
+template <typename S>
+__device__ inline void load_f8(const void* src, int64_t i, float* f);
+template <>
+__device__ inline void load_f8<uint16_t>(const void* src, int64_t i, float* f) {
+    const s16x8 v = ld16_stream(static_cast<const uint16_t*>(src) + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = BF16::to_float((uint16_t)v[e]);
+}
+template <>
+__device__ inline void load_f8<float>(const void* src, int64_t i, float* f) {
+    const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(src) + i);
+    const f32x4 a = __builtin_nontemporal_load(p), b = __builtin_nontemporal_load(p + 1);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        f[e] = a[e];
+        f[4 + e] = b[e];
+    }
+}
+template <typename S>
+__device__ inline float scaled(float x, float u) {
+    if constexpr (sizeof(S) == 2) return BF16::to_float(BF16::from_float(x * u));
+    else return x * u;
+}
+template <typename S, int DST>
+__global__ __launch_bounds__(256) void scale_cast_kernel(mykfa_scale_params p) {
+    const float u = *p.factor;
+    const int64_t chunks = p.n / 8;
+    for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < chunks; c += (int64_t)gridDim.x * 256) {
+        float f[8];
+        load_f8<S>(p.src, c * 8, f);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] = scaled<S>(f[e], u);
+        if constexpr (DST == MYKFA_FP32) {
+            f32x4* d = reinterpret_cast<f32x4*>(static_cast<float*>(p.dst) + c * 8);
+            __builtin_nontemporal_store(f32x4{f[0], f[1], f[2], f[3]}, d);
+            __builtin_nontemporal_store(f32x4{f[4], f[5], f[6], f[7]}, d + 1);
+        } else {
+            using T = std::conditional_t<DST == MYKFA_BF16, BF16, FP16>;
+            const u32x4 w = {T::pack2(f[0], f[1]), T::pack2(f[2], f[3]), T::pack2(f[4], f[5]), T::pack2(f[6], f[7])};
+            __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(p.dst) + c * 8));
+        }
+    }
+    if (blockIdx.x == 0 && (int64_t)threadIdx.x < p.n % 8) {
+        const int64_t i = chunks * 8 + threadIdx.x;
+        const float x = sizeof(S) == 2 ? BF16::to_float(static_cast<const uint16_t*>(p.src)[i])
+                                       : static_cast<const float*>(p.src)[i];
+        const float y = scaled<S>(x, u);
+        if constexpr (DST == MYKFA_FP32) static_cast<float*>(p.dst)[i] = y;
+        else if constexpr (DST == MYKFA_BF16) static_cast<uint16_t*>(p.dst)[i] = BF16::from_float(y);
+        else static_cast<uint16_t*>(p.dst)[i] = FP16::from_float(y);
+    }
+}
+template <typename S>
+void scale_launch(const mykfa_scale_params& p, hipStream_t s) {
+    const long long blocks = (p.n / 8 + 256 * 4 - 1) / (256 * 4);  // four chunks a lane
+    const dim3 grid((unsigned)(blocks < 1 ? 1 : blocks < 65536 ? blocks : 65536)), block(256);
+    if (p.dst_dtype == MYKFA_FP32) hipLaunchKernelGGL((scale_cast_kernel<S, MYKFA_FP32>), grid, block, 0, s, p);
+    else if (p.dst_dtype == MYKFA_BF16) hipLaunchKernelGGL((scale_cast_kernel<S, MYKFA_BF16>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((scale_cast_kernel<S, MYKFA_FP16>), grid, block, 0, s, p);
 }
 
 }  // namespace
@@ -318,6 +458,17 @@ hipError_t ce_dtype(const mykfa_ce_params& p, hipStream_t s) {
 hipError_t launch_ce_rows(const mykfa_ce_params& p, hipStream_t stream) {
     if (p.dtype == MYKFA_BF16) return ce_dtype<BF16>(p, stream);
     return ce_dtype<FP16>(p, stream);
+}
+
+hipError_t launch_ce_loss(const mykfa_ce_loss_params& p, hipStream_t stream) {
+    hipLaunchKernelGGL(ce_loss_kernel, dim3(1), dim3(kSumThreads), 0, stream, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_scale(const mykfa_scale_params& p, hipStream_t stream) {
+    if (p.src_dtype == MYKFA_FP32) scale_launch<float>(p, stream);
+    else scale_launch<uint16_t>(p, stream);
+    return hipGetLastError();
 }
 
 }  // namespace mykfa

@@ -138,13 +138,6 @@ __device__ inline void wave_fence() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// Results are not read again by this launch: stored past the L2, whose panels they would evict
-// (2048 x 65536 x 1024: 285 -> 260 us).
-template <typename V, typename E>
-__device__ inline void store16(E* c, V w) {
-    __builtin_nontemporal_store(w, reinterpret_cast<V*>(c));
-}
-
 // 8 elements of a row of which `left` exist.
 __device__ inline void store8(uint16_t* c, s16x8 w, int left, bool vec) {
     if (left >= 8) {
@@ -374,7 +367,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
                         if (full || (m < p.m && n < n_end)) {
                             uint16_t* c = cb + (int64_t)m * p.c_rs + n;
                             if constexpr (OUT == OUT_SYM) store8(c, y, n_end - n, p.c_vec);
-                            else store16(c, y);
+                            else st16(c, y);
                         }
                     }
                     if (OUT == OUT_SYM && t.m0 != t.n0) {
@@ -440,7 +433,10 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
                     f32x4 w = *reinterpret_cast<const f32x4*>(trf + r % 16 * 32 + ((ch ^ (r & 7)) << 2));
                     if (add) w += old[q] * p.beta;
                     float* c = at(x, q);
-                    if (c) store16(c, w);
+                    // Past the caches, whose panels the sums would evict (285 -> 260 us for 268 MB written
+                    // once); bf16 results are the next launch's input and stay (the fused head 7837 against
+                    // 7599 us with them past the caches).
+                    if (c) __builtin_nontemporal_store(w, reinterpret_cast<f32x4*>(c));
                 }
             }
         }

@@ -50,6 +50,8 @@ hipError_t launch_gate(const mykfa_gate_params& p, bool backward, hipStream_t st
 
 // Cross-entropy rows of the fused linear + cross-entropy (fused_ce.hip).
 hipError_t launch_ce_rows(const mykfa_ce_params& p, hipStream_t stream);
+hipError_t launch_ce_loss(const mykfa_ce_loss_params& p, hipStream_t stream);
+hipError_t launch_scale(const mykfa_scale_params& p, hipStream_t stream);
 
 // Batched matrix products and Muon's SYRK (gemm.hip); its Newton-Schulz iteration (muon.hip).
 size_t gemm_workspace_bytes(const mykfa_gemm_params& p);

@@ -13,10 +13,11 @@ gfx950 CE row kernel (csrc/fused_ce.hip, through the C ABI) with d loss / d logi
 next two GEMMs fold into the hidden and weight gradients at once. As in the reference the
 gradient is computed during the forward pass, so the loss is backpropagated exactly once.
 
-The three products per chunk are plain library GEMMs (torch.matmul on ROCm = hipBLASLt). The
-weight gradient accumulates in fp32 inside the GEMM (beta = 1, fp32 output) instead of rounding
-each chunk's bf16 product before an fp32 add (fused_ce.py:89): one pass over the fp32
-gradient per chunk instead of three, and no bf16 rounding of the partial sums.
+The products are libmykfa.so's (csrc/gemm.hip) where the hidden size is a multiple of 8, else
+torch.matmul's. The weight gradient accumulates in fp32 inside its product instead of rounding each
+chunk's bf16 product before an fp32 add (fused_ce.py:89), and takes the tokens of several chunks at
+once: the chunks' d logits are kept in a buffer of up to _KEEP_BYTES (one chunk where that, or the
+device's memory, holds no more).
 """
 
 from __future__ import annotations
@@ -29,6 +30,7 @@ from torch import Tensor
 
 from . import _lib
 from .flash_attn import _DeviceGuard, _dtype_code, _same_device, _stream
+from .gemm import gemm, usable
 
 
 def _ce_rows(logits: Tensor, targets: Tensor, ce: Tensor, lse: Tensor, scale: float, z_coef: float,
@@ -52,23 +54,52 @@ def _chunk_spans(n: int, size: int) -> list[tuple[int, int]]:
     return [(lo, min(lo + size, n)) for lo in range(0, n, size)]
 
 
+# d logits kept for one weight-gradient product. Its fp32 sums are read and written once per
+# product: 65536 x 1024 over 8192 tokens takes 4 x 335 us in chunks of 2048 with the sums read back,
+# 990 at once; the whole head over 16384 tokens 8137 us with one chunk kept, 7746, 7599 and 7506 with
+# two, four and eight.
+_KEEP_BYTES = 1 << 30
+
+
 def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: float, z_coef: float,
                         ignore_index: int, chunk_size: int) -> tuple[Tensor, Tensor, Tensor]:
     """One pass over the tokens in chunks. Returns (row_stats, d_hidden, d_weight):
     row_stats[0] / row_stats[1] are every token's cross-entropy and natural-log LSE (fp32),
     d_hidden (bf16) and d_weight (fp32) the gradients of the loss for an upstream gradient of 1.
 
-    Per chunk: the logits GEMM writes a (rows, vocab) bf16 block, the gfx950 row kernel turns
+    Per chunk: the logits product writes a (rows, vocab) bf16 block, the gfx950 row kernel turns
     that block into d loss / d logits in place while producing the row statistics, and the
-    same block then feeds the two gradient GEMMs. d_weight is accumulated in fp32 by the
-    GEMM (beta = 1) so no partial sum is ever rounded to bf16."""
+    same block then feeds the two gradient products. d_weight is accumulated in fp32 by the
+    product (beta = 1) so no partial sum is ever rounded to bf16."""
     dev = hidden.device
     tokens, width = hidden.shape
+    vocab = weight.shape[0]
     w16 = weight if weight.dtype == torch.bfloat16 else weight.to(torch.bfloat16)
     row_stats = torch.empty((2, tokens), dtype=torch.float32, device=dev)
     d_hidden = torch.empty((tokens, width), dtype=torch.bfloat16, device=dev)
-    d_weight = torch.zeros(weight.shape, dtype=torch.float32, device=dev)
     tgt = targets if targets.dtype == torch.int64 else targets.to(torch.int64)
+    stride = (vocab + 7) // 8 * 8
+    if width % 8 == 0 and width > 0 and vocab > 0 and tokens > 0 and max(stride, width) < 1 << 22:
+        h16 = hidden if hidden.dtype == torch.bfloat16 else hidden.to(torch.bfloat16)
+        h16, w16 = (x if usable(x) else x.contiguous() for x in (h16, w16))
+        d_weight = torch.empty((vocab, width), dtype=torch.float32, device=dev)
+        chunk = min(chunk_size, tokens)
+        kept = max(1, min(_KEEP_BYTES // (2 * chunk * stride), (tokens + chunk - 1) // chunk)) * chunk
+        try:
+            blocks = torch.empty((kept, stride), dtype=torch.bfloat16, device=dev)
+        except torch.OutOfMemoryError:
+            kept = chunk
+            blocks = torch.empty((kept, stride), dtype=torch.bfloat16, device=dev)
+        for first, last in _chunk_spans(tokens, kept):
+            for lo, hi in _chunk_spans(last - first, chunk):
+                block, a, b = blocks[lo:hi, :vocab], first + lo, first + hi
+                gemm(h16[a:b], w16, block, b - a, vocab, width, b_transposed=True)
+                _ce_rows(block, tgt[a:b], row_stats[0, a:b], row_stats[1, a:b], scale, z_coef, ignore_index)
+                gemm(block, w16, d_hidden[a:b], b - a, width, vocab)
+            gemm(blocks, h16[first:last], d_weight, vocab, width, last - first, a_transposed=True,
+                 beta=0.0 if first == 0 else 1.0)
+        return row_stats, d_hidden, d_weight
+    d_weight = torch.zeros(weight.shape, dtype=torch.float32, device=dev)
     for lo, hi in _chunk_spans(tokens, chunk_size):
         h16 = hidden[lo:hi]
         if h16.dtype != torch.bfloat16:
@@ -78,6 +109,37 @@ def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: 
         torch.mm(block, w16, out=d_hidden[lo:hi])
         _accumulate_fp32(d_weight, block.t(), h16)
     return row_stats, d_hidden, d_weight
+
+
+_SCALE_DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16, torch.float32: _lib.DTYPE_FP32}
+
+
+def _loss_of(row_stats: Tensor, scale: float, z_coef: float) -> tuple[Tensor, Tensor, Tensor]:
+    """(loss, ce_sum, z_sum) of the tokens' statistics."""
+    if row_stats.shape[1] > 1 << 17:  # more than one workgroup should sum
+        ce_sum = row_stats[0].sum()
+        z_sum = torch.dot(row_stats[1], row_stats[1])
+        return torch.add(ce_sum, z_sum, alpha=z_coef) * scale, ce_sum, z_sum
+    out = tuple(row_stats.new_empty(()) for _ in range(3))
+    ce = row_stats.data_ptr()
+    p = _lib.CeLossParams(ce, ce + 4 * row_stats.shape[1], *(x.data_ptr() for x in out), row_stats.shape[1], scale, z_coef)
+    with _DeviceGuard(row_stats.device):
+        _lib.check(_lib.lib().mykfa_ce_loss(ctypes.byref(p), _stream(row_stats.device)))
+    return out
+
+
+def _scaled(grad: Tensor, upstream: Tensor, dtype: torch.dtype) -> Tensor:
+    """grad * upstream, rounded to grad's type, as dtype."""
+    if (dtype not in _SCALE_DTYPES or upstream.dtype != torch.float32 or upstream.device != grad.device
+            or torch.is_grad_enabled() or torch._C._functorch.is_functorch_wrapped_tensor(upstream)
+            or torch._C._functorch.is_legacy_batchedtensor(upstream)):
+        return grad.mul(upstream).to(dtype)  # a gradient of the gradient, or a mapped one, goes through torch
+    out = torch.empty_like(grad, dtype=dtype)
+    p = _lib.ScaleParams(grad.data_ptr(), out.data_ptr(), upstream.data_ptr(), grad.numel(), _SCALE_DTYPES[grad.dtype],
+                         _SCALE_DTYPES[dtype])
+    with _DeviceGuard(grad.device):
+        _lib.check(_lib.lib().mykfa_scale(ctypes.byref(p), _stream(grad.device)))
+    return out
 
 
 class _LinearCrossEntropy(torch.autograd.Function):
@@ -91,18 +153,17 @@ class _LinearCrossEntropy(torch.autograd.Function):
         with torch.autocast(device_type="cuda", enabled=False), _DeviceGuard(hidden.device):
             row_stats, d_hidden, d_weight = _loss_and_gradients(hidden, weight, targets, scale, z_coef,
                                                                 ignore_index, chunk_size)
-        ce_sum = row_stats[0].sum()
-        z_sum = torch.dot(row_stats[1], row_stats[1])
+        loss, ce_sum, z_sum = _loss_of(row_stats, scale, z_coef)
         ctx.save_for_backward(d_hidden, d_weight)
         ctx.grad_dtypes = (hidden.dtype, weight.dtype)
         ctx.mark_non_differentiable(ce_sum, z_sum)
-        return torch.add(ce_sum, z_sum, alpha=z_coef) * scale, ce_sum, z_sum
+        return loss, ce_sum, z_sum
 
     @staticmethod
     def backward(ctx, upstream, _unused_ce, _unused_z):  # pyright: ignore[reportIncompatibleMethodOverride]
         d_hidden, d_weight = ctx.saved_tensors
         hidden_dtype, weight_dtype = ctx.grad_dtypes
-        return (d_hidden.mul(upstream).to(hidden_dtype), d_weight.mul(upstream).to(weight_dtype),
+        return (_scaled(d_hidden, upstream, hidden_dtype), _scaled(d_weight, upstream, weight_dtype),
                 None, None, None, None, None)
 
 

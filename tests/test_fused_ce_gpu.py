@@ -18,7 +18,7 @@ import pytest
 import torch
 
 from _util import storage_ulp
-from myk_llm_amd import _lib
+from myk_llm_amd import _lib, fused_ce
 from myk_llm_amd.fused_ce import _ce_rows, fused_linear_cross_entropy
 from oracle import fused_ce as oc
 
@@ -181,3 +181,55 @@ def test_model_head_shape():
         # the reference's gradient tolerance (tests/test_fused_ce.py:37-38) scaled to the
         # gradient's magnitude (1 / normalizer here, vs 1 / 123 there)
         torch.testing.assert_close(got.float(), ref, rtol=2e-2, atol=2e-2 * ref.abs().max().item())
+
+
+@pytest.mark.parametrize("rows, vocab, stride", [(5, 1001, 1008), (3, 4095, 4096), (2, 7, 8), (4, 65535, 65544), (3, 32003, 32008)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_rows_with_a_vocabulary_tail(rows, vocab, stride, dtype):
+    """Padded rows whose vocabulary is no multiple of 8 against the streaming kernel's elementwise
+    result on unpadded rows (the same formula; one rounding of the 16-bit result apart), ignored
+    and last-column targets included; the pad columns stay untouched."""
+    g = torch.Generator().manual_seed(vocab)
+    x = (4 * torch.randn(rows, vocab, generator=g)).to(dtype).cuda()
+    targets = torch.randint(0, vocab, (rows,), generator=g).cuda()
+    targets[0], targets[-1] = vocab - 1, -100
+    padded = torch.full((rows, stride), 7.0, dtype=dtype, device="cuda")
+    padded[:, :vocab] = x
+    plain = torch.empty(rows * (vocab | 1) + rows, dtype=dtype, device="cuda").as_strided((rows, vocab), (vocab | 1, 1))
+    plain.copy_(x)
+    got, exp = (torch.empty(2, rows, device="cuda") for _ in range(2))
+    fused_ce._ce_rows(padded[:, :vocab], targets, got[0], got[1], 0.5, 1e-3, -100)
+    fused_ce._ce_rows(plain, targets, exp[0], exp[1], 0.5, 1e-3, -100)
+    torch.testing.assert_close(got, exp, rtol=1e-5, atol=1e-5)
+    ulp = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    torch.testing.assert_close(padded[:, :vocab].float(), plain.float(), rtol=ulp, atol=2.0 ** -24)
+    assert (padded[:, vocab:] == 7).all()
+
+
+@pytest.mark.parametrize("tokens, width, vocab, chunk, keep", [(100, 72, 1003, 33, 1 << 30), (100, 72, 1003, 33, 1), (517, 64, 264, 128, 2 * 264 * 2 * 128)])
+@pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)])
+def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, dtypes):
+    """Any number of chunks per weight-gradient product gives the reference's loss and gradients."""
+    monkeypatch.setattr(fused_ce, "_KEEP_BYTES", keep)
+    g = torch.Generator().manual_seed(tokens)
+    hidden = torch.randn(tokens, width, generator=g).to(torch.bfloat16).to(dtypes[0]).cuda().requires_grad_()
+    weight = (0.1 * torch.randn(vocab, width, generator=g)).to(torch.bfloat16).to(dtypes[1]).cuda().requires_grad_()
+    targets = torch.randint(0, vocab, (tokens,), generator=g).cuda()
+    targets[::7] = -100
+    n = float((targets != -100).sum())
+    loss, ce_sum, z_sum = fused_ce.fused_linear_cross_entropy(hidden, weight, targets, n, 1e-3, chunk_size=chunk)
+    (3.0 * loss).backward()
+    h, w = (x.detach().double().requires_grad_() for x in (hidden, weight))
+    logits = h @ w.t()
+    lse = torch.logsumexp(logits, -1)
+    valid = targets != -100
+    ce = (lse - logits.gather(1, targets.clamp_min(0)[:, None])[:, 0])[valid].sum()
+    z = lse[valid].square().sum()
+    exp = (ce + 1e-3 * z) / n
+    (3.0 * exp).backward()
+    for got, want in ((loss, exp), (ce_sum, ce), (z_sum, z)):
+        torch.testing.assert_close(got.double(), want, rtol=2e-3, atol=0)
+    for got, want in ((hidden.grad, h.grad), (weight.grad, w.grad)):
+        assert got.dtype in dtypes
+        err = (got.double() - want).norm() / want.norm()
+        assert err < 1e-2, err  # bf16 logits and gradients: 2^-8 each

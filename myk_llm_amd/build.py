@@ -1,4 +1,5 @@
-"""Build libmykfa.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc.
+"""Build libmykfa.so (the gfx950 HIP kernels + C ABI) in-tree with hipcc, and _host.so (the native
+host path of the attention calls, csrc/host.cpp) with the host compiler against torch's headers.
 
     python -m myk_llm_amd.build            # compile every csrc/*.hip, link myk_llm_amd/libmykfa.so
 
@@ -13,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libmykfa.so"
+HOST = PKG / "_host.so"
 ARCH = os.environ.get("MYKFA_ARCH", "gfx950")
 
 # Packed-FP32 instruction selection (v_pk_*_f32) is disabled for every HIP object: some of
@@ -59,6 +62,24 @@ def _compile(hipcc: str, src: Path) -> Path:
     return obj
 
 
+def _build_host() -> None:
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    tmp = HOST.with_suffix(".so.tmp")
+    rocm = Path(_hipcc()).resolve().parent.parent
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{p}" for p in include_paths()), f"-I{sysconfig.get_paths()['include']}", f"-I{rocm / 'include'}",
+           str(CSRC / "host.cpp"), "-o", str(tmp), *(f"-L{p}" for p in library_paths()),
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on host.cpp:\n{res.stderr}")
+    os.replace(tmp, HOST)
+
+
 def build(verbose: bool = True) -> Path:
     hipcc = _hipcc()
     BUILD.mkdir(exist_ok=True)
@@ -66,8 +87,10 @@ def build(verbose: bool = True) -> Path:
     if not sources:
         raise RuntimeError(f"no HIP sources under {CSRC}")
     workers = min(len(sources), max(1, min(8, os.cpu_count() or 1)))
-    with concurrent.futures.ThreadPoolExecutor(workers) as pool:
+    with concurrent.futures.ThreadPoolExecutor(workers + 1) as pool:
+        host = pool.submit(_build_host)
         objs = list(pool.map(lambda s: _compile(hipcc, s), sources))
+        host.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -75,7 +98,7 @@ def build(verbose: bool = True) -> Path:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB)
     if verbose:
-        print(f"built {LIB} from {len(sources)} sources for {ARCH}")
+        print(f"built {LIB} from {len(sources)} sources for {ARCH}, and {HOST}")
     return LIB
 
 

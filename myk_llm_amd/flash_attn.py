@@ -443,6 +443,30 @@ class _FlashAttn(torch.autograd.Function):
         return dq, dk, dv, None, None, None, None, None, None, None, None
 
 
+# --- the native host path (csrc/host.cpp) ---------------------------------------------------
+
+_host = None
+_HOST_ENTRIES = ("fwd", "fwd_workspace_size", "fwd_ws", "bwd", "bwd_workspace_per_kv_head", "decode",
+                 "decode_num_splits", "decode_workspace_size", "kv_append")
+
+
+def _native():
+    """The extension that makes the plain calls (GPU tensors as the kernels read them): it answers
+    NotImplemented to every other, which then takes the code below."""
+    global _host
+    if _host is None:
+        L = _lib.lib()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise RuntimeError("myk_llm_amd/_host.so is missing or does not load: build it first "
+                               "(python -m myk_llm_amd.build)") from e
+        mod.setup(*(ctypes.cast(getattr(L, f"mykfa_{n}"), ctypes.c_void_p).value for n in _HOST_ENTRIES),
+                  _lib.check, _backward_launch)
+        _host = mod
+    return _host
+
+
 # --- public API (flash_attn.py:442-490) ----------------------------------------------------
 
 
@@ -452,6 +476,10 @@ def flash_attn_func(
 ):
     """Attention over a dense batch: q is (B, Sq, Hq, D) and k, v are (B, Sk, Hkv, D) with Hq a
     multiple of Hkv. Returns O shaped like q (and the base-2 LSE with return_softmax_lse)."""
+    if q.is_cuda and not _compiling():
+        r = _native().attention(q, k, v, None, None, 0, 0, causal, window_size, softmax_scale, return_softmax_lse)
+        if r is not NotImplemented:
+            return r
     _check(q, k, v)
     q, k, v = (_last_dim_contiguous(x) for x in (q, k, v))
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(q.shape[-1])
@@ -468,6 +496,11 @@ def flash_attn_varlen_func(
     owns query rows [cu_seqlens_q[b], cu_seqlens_q[b + 1]) and key rows likewise from
     cu_seqlens_k (int32 offsets on q's GPU). max_seqlen_q / max_seqlen_k bound the longest
     document and only size the launch grid."""
+    if q.is_cuda and not _compiling():
+        r = _native().attention(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal, window_size,
+                                softmax_scale, return_softmax_lse)
+        if r is not NotImplemented:
+            return r
     _check(q, k, v)
     _same_device(q.device, cu_seqlens_q=cu_seqlens_q, cu_seqlens_k=cu_seqlens_k)
     q, k, v = (_last_dim_contiguous(x) for x in (q, k, v))
@@ -489,6 +522,11 @@ def flash_attn_with_kvcache(
     caller, and no gradient flows. A position at or past the capacity is not written (the
     reference's index write would fault there) and the attended length is clipped to the
     capacity."""
+    if k is not None and v is not None and q.is_cuda and not _compiling():
+        r = _native().kvcache(q, k_cache, v_cache, k, v, cache_seqlens, causal, window_size, softmax_scale,
+                              return_softmax_lse)
+        if r is not NotImplemented:
+            return r
     _check(q, k_cache, v_cache)
     if k_cache.stride(-1) != 1 or v_cache.stride(-1) != 1:
         raise ValueError("the caches need a contiguous last dimension")

@@ -1,0 +1,154 @@
+"""The native host path against the Python one it stands in for: the same bits for every form that
+it accepts, and the same answer from autograd where it is looked at from outside (hooks on saved
+tensors, a second backward, gradients of gradients, mapped and forward-mode gradients)."""
+
+import pytest
+import torch
+
+from myk_llm_amd import flash_attn as fa
+from myk_llm_amd import flash_attn_func, flash_attn_varlen_func, flash_attn_with_kvcache
+
+pytestmark = pytest.mark.gpu
+
+
+class _Never:
+    @staticmethod
+    def attention(*a):
+        return NotImplemented
+
+    kvcache = attention
+
+
+def _both(monkeypatch, call):
+    got = call()
+    with monkeypatch.context() as m:
+        m.setattr(fa, "_host", _Never)
+        return got, call()
+
+
+def _same(got, exp):
+    assert len(got) == len(exp)
+    for a, b in zip(got, exp):
+        assert (a is None) == (b is None) and (a is None or (a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b)))
+        assert a is None or (a.requires_grad == b.requires_grad and a.stride() == b.stride())
+
+
+def _qkv(g, lead, hq, hk, d, dtype, form):
+    def make(h):
+        if form == "sliced":  # one of a wider projection's parts
+            x = torch.randn(*lead, h + 2, d, generator=g)[..., 1:1 + h, :]
+            return x.to(dtype).cuda()
+        if form == "heads_first":
+            return torch.randn(*lead[:-1], h, lead[-1], d, generator=g).to(dtype).cuda().transpose(-3, -2)
+        if form == "unaligned":  # not what the kernels read: copied by the Python path
+            return torch.randn(*lead, h, d + 3, generator=g).to(dtype).cuda()[..., 3:]
+        return torch.randn(*lead, h, d, generator=g).to(dtype).cuda()
+
+    return make(hq), make(hk), make(hk)
+
+
+@pytest.mark.parametrize("form", ["plain", "sliced", "heads_first", "unaligned"])
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("d, dtype, needs", [(64, torch.bfloat16, "qkv"), (128, torch.float16, "qkv"), (32, torch.bfloat16, "k"),
+                                             (64, torch.bfloat16, "")])
+@pytest.mark.parametrize("with_lse", [False, True])
+def test_attention_bits(monkeypatch, form, packed, d, dtype, needs, with_lse):
+    g = torch.Generator().manual_seed(d)
+    q, k, v = _qkv(g, (150,) if packed else (2, 75), 4, 2, d, dtype, form)
+    for n, x in (("q", q), ("k", k), ("v", v)):
+        x.requires_grad_(n in needs)
+    cu = torch.tensor([0, 31, 150], dtype=torch.int32, device="cuda")
+    dout = torch.randn(4, q.shape[-3] if packed else 75, d, generator=g).to(dtype).cuda().transpose(0, 1)
+    dout = dout if packed else dout.expand(2, 75, 4, d)
+
+    def call():
+        kw = dict(causal=True, window_size=(40, 0), softmax_scale=0.2, return_softmax_lse=with_lse)
+        r = flash_attn_varlen_func(q, k, v, cu, cu, 119, 119, **kw) if packed else flash_attn_func(q, k, v, **kw)
+        out = r[0] if with_lse else r
+        ins = [x for x in (q, k, v) if x.requires_grad]
+        return (*(r if with_lse else (r,)), *(torch.autograd.grad(out, ins, dout) if ins else ()))
+
+    _same(*_both(monkeypatch, call))
+
+
+@pytest.mark.parametrize("nq, lens, with_lse", [(1, [0, 200], False), (16, [3, 77], True), (17, [0, 200], True), (40, [250, 1], False)])
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+def test_kvcache_bits(monkeypatch, nq, lens, with_lse, index):
+    g = torch.Generator().manual_seed(nq)
+    q, k, v = _qkv(g, (2, nq), 8, 2, 64, torch.bfloat16, "plain")
+    caches = torch.randn(2, 2, 256, 2, 64, generator=g).to(torch.bfloat16).cuda()
+    cl = torch.tensor(lens, dtype=index, device="cuda")
+
+    def call():
+        kc, vc = caches[0].clone(), caches[1].clone()
+        r = flash_attn_with_kvcache(q, kc, vc, k, v, cache_seqlens=cl, causal=True, return_softmax_lse=with_lse)
+        return (*(r if with_lse else (r,)), kc, vc)
+
+    _same(*_both(monkeypatch, call))
+
+
+def _error(call):
+    try:
+        call()
+    except Exception as e:  # noqa: BLE001
+        return type(e)
+    return None
+
+
+def test_refusals_and_autograd_from_outside(monkeypatch):
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (x.requires_grad_() for x in _qkv(g, (2, 40), 4, 2, 64, torch.bfloat16, "plain"))
+    grad = torch.randn(2, 40, 4, 64, generator=g).to(torch.bfloat16).cuda()
+
+    def second_backward():
+        out = flash_attn_func(q, k, v)
+        out.backward(grad)
+        out.backward(grad)
+
+    def changed_in_place():
+        x = q.clone()
+        out = flash_attn_func(x, k, v)
+        x.mul_(2)
+        out.backward(grad)
+
+    def mapped():
+        out = flash_attn_func(q, k, v)
+        torch.autograd.grad(out, q, torch.stack([grad, grad]), is_grads_batched=True)
+
+    def functional():
+        torch.func.grad(lambda x: flash_attn_func(x, k, v).float().sum())(q.detach())
+
+    def forward_mode():
+        with torch.autograd.forward_ad.dual_level():
+            flash_attn_func(torch.autograd.forward_ad.make_dual(q.detach(), grad), k, v)
+
+    def wrong_heads():
+        flash_attn_func(q[:, :, :3], k, v)
+
+    def wrong_dtype():
+        flash_attn_func(q, k.half(), v)
+
+    def host_keys():
+        flash_attn_func(q, k.cpu(), v)
+
+    for call in (second_backward, changed_in_place, mapped, functional, forward_mode, wrong_heads, wrong_dtype, host_keys):
+        got, exp = _both(monkeypatch, lambda call=call: _error(call))
+        assert got is exp and got is not None, (call.__name__, got, exp)
+
+    def hooked():
+        seen = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda x: (seen.append(tuple(x.shape)), x * 1)[1], lambda x: x):
+            out = flash_attn_func(q, k, v, causal=True)
+        return (torch.tensor(len(seen)), *torch.autograd.grad(out, (q, k, v), grad))
+
+    def twice():
+        out = flash_attn_func(q, k, v)
+        return torch.autograd.grad(out, (q, k, v), grad, create_graph=True)
+
+    def unused():
+        out, lse = flash_attn_func(q, k, v, return_softmax_lse=True)
+        return (*torch.autograd.grad(out.float().sum(), (q,), retain_graph=True), torch.tensor(out.requires_grad),
+                torch.tensor(lse.requires_grad))
+
+    for call in (hooked, twice, unused):
+        _same(*_both(monkeypatch, call))

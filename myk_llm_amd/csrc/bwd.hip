@@ -1259,6 +1259,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dq_kernel(BwdArgs a) {
     constexpr int KB = BN / 16;
     using Ring = TileRing<D, BN, 2, NW>;
     __shared__ __attribute__((aligned(16))) uint16_t smem[STAGES][2][BN * D];
+    __shared__ __attribute__((aligned(16))) uint16_t rows_out[D >= 32 ? NW : 1][2048];  // store_rows32
 
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int l32 = lane & 31, g = lane >> 5;
@@ -1427,19 +1428,20 @@ __global__ __launch_bounds__(NW * 64) void bwd_dq_kernel(BwdArgs a) {
             }
     }
 
-    if (q_ok) {
+    if constexpr (D >= 32) {
+        uint16_t* dqp = a.dq + (int64_t)b * a.dqbs + (qs.tok0 + s0) * a.dqts + (int64_t)h * a.dqhs;
+        store_rows32<T, DB>(rows_out[wave], acc, a.sm_scale, dqp, a.dqts, q_len - s0, lane);
+    } else if (q_ok) {
         uint16_t* dqp = a.dq + (int64_t)b * a.dqbs + (qs.tok0 + qi) * a.dqts + (int64_t)h * a.dqhs;
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int rq = 0; rq < 4; ++rq) {
-                const int d0 = 32 * db + 8 * rq + 4 * g;
-                if (d0 < D) {
-                    u32x2 w = {T::pack2(acc[db][4 * rq] * a.sm_scale, acc[db][4 * rq + 1] * a.sm_scale),
-                               T::pack2(acc[db][4 * rq + 2] * a.sm_scale, acc[db][4 * rq + 3] * a.sm_scale)};
-                    *reinterpret_cast<u32x2*>(dqp + d0) = w;
-                }
+        for (int rq = 0; rq < 4; ++rq) {
+            const int d0 = 8 * rq + 4 * g;
+            if (d0 < D) {
+                u32x2 w = {T::pack2(acc[0][4 * rq] * a.sm_scale, acc[0][4 * rq + 1] * a.sm_scale),
+                           T::pack2(acc[0][4 * rq + 2] * a.sm_scale, acc[0][4 * rq + 3] * a.sm_scale)};
+                *reinterpret_cast<u32x2*>(dqp + d0) = w;
             }
+        }
     }
 }
 
@@ -1597,22 +1599,13 @@ __device__ __forceinline__ void dq_ds_block(const BwdArgs& a, int logical) {
         }
     }
 
-    // dQ^T rows = d (registers), columns = queries (lanes): 8-byte stores of 4 consecutive d.
+    // The ring's last stage has been read by every wave: its memory takes the stores' exchange.
+    barrier_lds();
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
-        const int qi = s_w + 32 * tt + l32;
-        if (qi >= q_len) continue;
-        uint16_t* dqp = a.dq + (int64_t)b * a.dqbs + (qs.tok0 + qi) * a.dqts + (int64_t)h * a.dqhs;
-#pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int rq = 0; rq < 4; ++rq) {
-                const int d0 = 32 * db + 8 * rq + 4 * g;
-                const f32x16& c = acc[tt][db];
-                u32x2 w = {T::pack2(c[4 * rq] * a.sm_scale, c[4 * rq + 1] * a.sm_scale),
-                           T::pack2(c[4 * rq + 2] * a.sm_scale, c[4 * rq + 3] * a.sm_scale)};
-                *reinterpret_cast<u32x2*>(dqp + d0) = w;
-            }
+        const int row0 = s_w + 32 * tt;
+        uint16_t* dqp = a.dq + (int64_t)b * a.dqbs + (qs.tok0 + row0) * a.dqts + (int64_t)h * a.dqhs;
+        store_rows32<T, DB>(&smem[0][0] + wave * 2048, acc[tt], a.sm_scale, dqp, a.dqts, q_len - row0, lane);
     }
 }
 

@@ -199,6 +199,48 @@ __device__ inline void barrier_lds() {
     __builtin_amdgcn_s_barrier();
 }
 
+// Lanes of one wave exchange data through LDS: its operations execute in order, but the compiler
+// must not carry a value across the other lanes' writes.
+__device__ inline void wave_fence() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Stores a wave's 32 x 32 DB result of 32x32 MFMAs (lane l32 = row, register 4 rq + i of block db =
+// column 32 db + 8 rq + 4 g + i), scaled and rounded, as rows base + r * stride, r < rows. Direct
+// stores would write 8 bytes of each of 32 rows at a time; through 4 KB of LDS (tr, this wave's own)
+// every store covers whole 128-byte lines (us, before and after for O and dQ: forward of 16384 packed
+// tokens, 16 heads of 128, 195 -> 187, of 4 x 8192 in a 1024 window 308 -> 299; their backwards
+// 626 -> 616 and 1020 -> 1005; 8248 tokens of 64, 46.8 -> 45.2 and 131 -> 128).
+template <typename T, int DB>
+__device__ inline void store_rows32(uint16_t* tr, const f32x16* acc, float scale, uint16_t* base, int64_t stride, int rows,
+                                    int lane) {
+    const int l32 = lane & 31, g = lane >> 5;
+    constexpr int NJ = DB < 2 ? 1 : 2;  // 32-column blocks at a time
+    static_assert(DB % NJ == 0, "whole passes");
+#pragma unroll
+    for (int dp = 0; dp < DB; dp += NJ) {
+        wave_fence();
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int rq = 0; rq < 4; ++rq) {
+                const f32x16& c = acc[dp + j];
+                const u32x2 w = {T::pack2(c[4 * rq] * scale, c[4 * rq + 1] * scale),
+                                 T::pack2(c[4 * rq + 2] * scale, c[4 * rq + 3] * scale)};
+                *reinterpret_cast<u32x2*>(tr + l32 * 64 + (((4 * j + rq) ^ (l32 & 7)) << 3) + 4 * g) = w;
+            }
+        wave_fence();
+        constexpr int CPR = 4 * NJ, RPI = 64 / CPR;  // chunks per row, rows per store
+#pragma unroll
+        for (int q = 0; q < 32 / RPI; ++q) {
+            const int r = RPI * q + lane / CPR, ch = lane % CPR;
+            const s16x8 x = *reinterpret_cast<const s16x8*>(tr + r * 64 + ((ch ^ (r & 7)) << 3));
+            if (r < rows) st16(base + r * stride + 32 * dp + 8 * ch, x);
+        }
+    }
+}
+
 // ---- asynchronous tile ring (buffer_load ... lds) ---------------------------------------
 // Rows [n0, n0 + ROWS) x D of NT tensors (16-bit, row stride in elements) are fetched straight
 // into a swizzled LDS tile by buffer loads with the LDS destination: lane l of a load writes

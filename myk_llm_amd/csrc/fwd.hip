@@ -84,6 +84,7 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     constexpr int KB = BN / 16;           // 16-key k-steps of O^T += V^T P^T
     using Ring = TileRing<D, BN, 2, NW>;  // K and V tiles
     __shared__ __attribute__((aligned(16))) uint16_t smem[STAGES][2][BN * D];
+    __shared__ __attribute__((aligned(16))) uint16_t rows_out[D >= 32 ? NW : 1][2048];  // store_rows32
 
     const int tid = __builtin_amdgcn_workitem_id_x();
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -313,19 +314,27 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     }
     const bool empty = l_tot == 0.f;
     const float inv = empty ? 0.f : 1.f / l_tot;
-    if (qi < q_len) {
-        uint16_t* op = a.o + (int64_t)b * a.obs + (qs.tok0 + qi) * a.ots + (int64_t)h * a.ohs;
+    if constexpr (D >= 32) {
+        uint16_t* op = a.o + (int64_t)b * a.obs + (qs.tok0 + s0) * a.ots + (int64_t)h * a.ohs;
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
+            for (int r = 0; r < 16; ++r) acc[db][r] *= inv;  // of this lane's row
+        store_rows32<T, DB>(rows_out[wave], acc, 1.f, op, a.ots, bs, lane);
+    }
+    if (qi < q_len) {
+        if constexpr (D < 32) {
+            uint16_t* op = a.o + (int64_t)b * a.obs + (qs.tok0 + qi) * a.ots + (int64_t)h * a.ohs;
+#pragma unroll
             for (int rq = 0; rq < 4; ++rq) {
-                const int d0 = 32 * db + 8 * rq + 4 * g;
+                const int d0 = 8 * rq + 4 * g;
                 if (d0 < D) {
-                    u32x2 w = {T::pack2(acc[db][4 * rq] * inv, acc[db][4 * rq + 1] * inv),
-                               T::pack2(acc[db][4 * rq + 2] * inv, acc[db][4 * rq + 3] * inv)};
+                    u32x2 w = {T::pack2(acc[0][4 * rq] * inv, acc[0][4 * rq + 1] * inv),
+                               T::pack2(acc[0][4 * rq + 2] * inv, acc[0][4 * rq + 3] * inv)};
                     *reinterpret_cast<u32x2*>(op + d0) = w;
                 }
             }
+        }
         if (g == 0) a.lse[(int64_t)h * a.lse_hs + qs.row0 + qi] = empty ? INFINITY : m_i + fast_log2(l_tot);
     }
 }

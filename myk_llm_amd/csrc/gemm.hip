@@ -131,13 +131,6 @@ struct Operand {
     }
 };
 
-// Lanes of one wave exchange data through LDS: its operations execute in order, but the compiler
-// must not carry a value across the other lanes' writes.
-__device__ inline void wave_fence() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // 8 elements of a row of which `left` exist.
 __device__ inline void store8(uint16_t* c, s16x8 w, int left, bool vec) {
     if (left >= 8) {

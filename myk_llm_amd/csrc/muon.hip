@@ -2,8 +2,8 @@
 // scaled (and, for tall matrices, transposed) bf16 copy, `steps` times three products (gemm.hip),
 // and the way back to the caller's layout.
 //   G = X X^T;  G2 = b G + c G G;  X' = a X + G2 X
-// X lives as (batch, M, K8) rows padded to a multiple of 8 with zeros, G and G2 as (batch, M, M8)
-// likewise, so that every product reads its operands as they are: at 5 x 776 x 328 the padded
+// X lives as (batch, M, K) rows a multiple of 64 apart, zero up to the next multiple of 8, G and G2
+// as (batch, M, M) likewise, so that every product reads its operands as they are: at 5 x 776 x 328 the padded
 // copies before each product were 20 launches of the 45.
 #include "common.h"
 #include "kernels.h"
@@ -16,6 +16,7 @@ constexpr int kMaxParts = 256;  // partial sums of squares per matrix
 constexpr int kT = 64;          // transpose tile
 
 int round8(int x) { return (x + 7) & ~7; }
+int row_stride(int x) { return (x + 63) & ~63; }  // rows start 128-byte lines
 
 // Sum over the workgroup in a fixed order; every thread gets it.
 __device__ inline float block_sum(float x, float* red) {
@@ -171,8 +172,8 @@ Sizes sizes_of(const mykfa_newton_schulz_params& p) {
     Sizes s;
     s.M = p.transposed ? p.cols : p.rows;
     s.K = p.transposed ? p.rows : p.cols;
-    s.x = (size_t)p.batch * s.M * round8(s.K) * 2;
-    s.g = (size_t)p.batch * s.M * round8(s.M) * 2;
+    s.x = (size_t)p.batch * s.M * row_stride(s.K) * 2;
+    s.g = (size_t)p.batch * s.M * row_stride(s.M) * 2;
     s.part = (size_t)p.batch * kMaxParts * sizeof(float);
     return s;
 }
@@ -187,7 +188,7 @@ size_t newton_schulz_bytes(const mykfa_newton_schulz_params& p) {
 
 hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, hipStream_t stream) {
     const Sizes z = sizes_of(p);
-    const int M = z.M, K = z.K, M8 = round8(M), K8 = round8(K);
+    const int M = z.M, K = z.K, M8 = round8(M), K8 = round8(K), Ms = row_stride(M), Ks = row_stride(K);
     char* w = static_cast<char*>(ws);
     uint16_t* xs[2] = {reinterpret_cast<uint16_t*>(w), reinterpret_cast<uint16_t*>(w + align256(z.x))};
     uint16_t* g = reinterpret_cast<uint16_t*>(w + 2 * align256(z.x));
@@ -200,7 +201,7 @@ hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, h
     c.in = static_cast<const uint16_t*>(p.x);
     c.out = xs[0];
     c.ibs = n; c.irs = p.cols;
-    c.obs = (int64_t)M * K8; c.ors = K8;
+    c.obs = (int64_t)M * Ks; c.ors = Ks;
     c.rows = p.rows; c.cols = p.cols; c.owidth = K8;
     c.eps = p.eps;
     if (!p.normalized) {
@@ -226,24 +227,25 @@ hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, h
     q.c_dtype = MYKFA_BF16;
     const uint16_t* x = xs[0];
     for (int i = 0; i < p.steps; ++i) {
-        uint16_t* next = i + 1 == p.steps && direct ? static_cast<uint16_t*>(p.out) : xs[(i + 1) & 1];
+        const bool last = i + 1 == p.steps && direct;
+        uint16_t* next = last ? static_cast<uint16_t*>(p.out) : xs[(i + 1) & 1];
         q.symmetric = 1;
         q.m = q.n = M;
-        q.a = x; q.a_batch_stride = (int64_t)M * K8; q.a_row_stride = K8; q.k = K8;
+        q.a = x; q.a_batch_stride = (int64_t)M * Ks; q.a_row_stride = Ks; q.k = K8;
         q.add = nullptr; q.alpha = 1.f; q.beta = 0.f;
-        q.c = g; q.c_batch_stride = (int64_t)M * M8; q.c_row_stride = M8;
+        q.c = g; q.c_batch_stride = (int64_t)M * Ms; q.c_row_stride = Ms;
         if ((e = launch_gemm(q, nullptr, stream)) != hipSuccess) return e;
-        q.a = g; q.a_batch_stride = (int64_t)M * M8; q.a_row_stride = M8; q.k = M8;
-        q.add = g; q.add_batch_stride = (int64_t)M * M8; q.add_row_stride = M8;
+        q.a = g; q.a_batch_stride = (int64_t)M * Ms; q.a_row_stride = Ms; q.k = M8;
+        q.add = g; q.add_batch_stride = (int64_t)M * Ms; q.add_row_stride = Ms;
         q.alpha = p.c; q.beta = p.b;
         q.c = g2;
         if ((e = launch_gemm(q, nullptr, stream)) != hipSuccess) return e;
         q.symmetric = 0;
         q.a = g2; q.m = M; q.n = K; q.k = M;
-        q.b = x; q.b_batch_stride = (int64_t)M * K8; q.b_row_stride = K8;
-        q.add = x; q.add_batch_stride = (int64_t)M * K8; q.add_row_stride = K8;
+        q.b = x; q.b_batch_stride = (int64_t)M * Ks; q.b_row_stride = Ks;
+        q.add = x; q.add_batch_stride = (int64_t)M * Ks; q.add_row_stride = Ks;
         q.alpha = 1.f; q.beta = p.a;
-        q.c = next; q.c_batch_stride = (int64_t)M * K8; q.c_row_stride = K8;
+        q.c = next; q.c_batch_stride = (int64_t)M * (last ? K8 : Ks); q.c_row_stride = last ? K8 : Ks;
         if ((e = launch_gemm(q, nullptr, stream)) != hipSuccess) return e;
         x = next;
     }
@@ -251,7 +253,7 @@ hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, h
     CopyArgs o{};
     o.in = x;
     o.out = static_cast<uint16_t*>(p.out);
-    o.ibs = (int64_t)M * K8; o.irs = K8;
+    o.ibs = (int64_t)M * Ks; o.irs = Ks;
     o.obs = n; o.ors = p.cols;
     o.rows = M; o.cols = K; o.owidth = p.transposed ? M : K;
     return copy(o, p.batch, p.transposed, stream);

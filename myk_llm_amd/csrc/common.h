@@ -241,6 +241,29 @@ __device__ inline void store_rows32(uint16_t* tr, const f32x16* acc, float scale
     }
 }
 
+// The same unscaled in fp32, as contiguous rows of 32 DB.
+template <int DB>
+__device__ inline void store_rows32_f32(float* tr, const f32x16* acc, float* base, int rows, int lane) {
+    const int l32 = lane & 31, g = lane >> 5;
+#pragma unroll
+    for (int db = 0; db < DB; ++db) {
+        wave_fence();
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+            const f32x16& c = acc[db];
+            *reinterpret_cast<f32x4*>(tr + l32 * 32 + (((2 * rq + g) ^ (l32 & 7)) << 2)) =
+                f32x4{c[4 * rq], c[4 * rq + 1], c[4 * rq + 2], c[4 * rq + 3]};
+        }
+        wave_fence();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int r = 8 * q + (lane >> 3), ch = lane & 7;
+            const f32x4 x = *reinterpret_cast<const f32x4*>(tr + r * 32 + ((ch ^ (r & 7)) << 2));
+            if (r < rows) *reinterpret_cast<f32x4*>(base + (int64_t)r * (32 * DB) + 32 * db + 4 * ch) = x;
+        }
+    }
+}
+
 // ---- asynchronous tile ring (buffer_load ... lds) ---------------------------------------
 // Rows [n0, n0 + ROWS) x D of NT tensors (16-bit, row stride in elements) are fetched straight
 // into a swizzled LDS tile by buffer loads with the LDS destination: lane l of a load writes

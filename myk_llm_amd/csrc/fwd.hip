@@ -297,19 +297,19 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     const float l_tot = sum_halves(l_i);
     if (SPLIT && parts > 1) {
         // A part: O unnormalized and (m, l), all fp32, for merge_kernel.
-        if (qi < q_len) {
-            const int64_t row = ((int64_t)bc.seq * (a.gz * a.hpw) + h) * a.seqlen_q + qi;
+        const int64_t row0 = ((int64_t)bc.seq * (a.gz * a.hpw) + h) * a.seqlen_q + s0;
+        if constexpr (D >= 32) {
+            store_rows32_f32<DB>(reinterpret_cast<float*>(rows_out[wave]), acc, a.ws_o + row0 * D, bs, lane);
+        } else if (qi < q_len) {
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int rq = 0; rq < 4; ++rq) {
-                    const int d0 = 32 * db + 8 * rq + 4 * g;
-                    if (d0 < D)
-                        *reinterpret_cast<f32x4*>(a.ws_o + row * D + d0) =
-                            f32x4{acc[db][4 * rq], acc[db][4 * rq + 1], acc[db][4 * rq + 2], acc[db][4 * rq + 3]};
-                }
-            if (g == 0) a.ws_ml[row] = f32x2{m_i, l_tot};
+            for (int rq = 0; rq < 4; ++rq) {
+                const int d0 = 8 * rq + 4 * g;
+                if (d0 < D)
+                    *reinterpret_cast<f32x4*>(a.ws_o + (row0 + l32) * D + d0) =
+                        f32x4{acc[0][4 * rq], acc[0][4 * rq + 1], acc[0][4 * rq + 2], acc[0][4 * rq + 3]};
+            }
         }
+        if (qi < q_len && g == 0) a.ws_ml[row0 + l32] = f32x2{m_i, l_tot};
         return;
     }
     const bool empty = l_tot == 0.f;
@@ -446,13 +446,14 @@ size_t fwd_split_bytes(const mykfa_fwd_params& p, int splits) {
 }
 
 // Parts per block when the blocks alone leave CUs idle (a prompt of some hundred tokens behind a
-// long cache: 389 queries of 16 heads are 52 workgroups of 100 key tiles each, 112.7 us on 256
-// CUs). Parts up to one workgroup per CU: measured (us, at 1 / 128 / 192 / 256 / 384 / 512 / 1024
-// workgroups) 112.7 / 66.7 / 50.7 / 45.4 / 42.3 / 51.4 / 59.4 there (bf16, D 128, 6389 keys),
-// 71.4 / 47.6 / 40.6 / 37.7 / 37.5 / 36.4 / 47.4 with 1000 queries of 8 heads on 3000 keys, 44.7 / 44.3 /
-// 32.6 / 32.5 / 30.1 / 31.3 / 34.6 with 2 x 1500 queries of 4 heads of 64 on 2000 keys: beyond one
-// workgroup per CU the partials cost what the shorter chains save. A block whose keys could fill
-// fewer than 16 tiles is not split: a 512 window took 18.4 us whole and 21.7 in two parts.
+// long cache: 389 queries of 16 heads are 52 workgroups of 100 key tiles each, 113 us on 256 CUs).
+// Up to 448 workgroups, just under two per CU (an XCD given more than its 64 slots runs a second
+// round). Measured (us, at 1 / 128 / 256 / 384 / 448 / 512 / 768 workgroups): 112.7 / 67.0 / 44.8 / 41.5 /
+// 40.2 / 49.1 / 48.3 there (bf16, D 128, 6389 keys), 70.5 / 46.8 / 37.3 / 36.0 / 34.6 / 35.5 / 35.4 with 1000
+// queries of 8 heads on 3000 keys, 44.6 / 44.2 / 32.6 / 30.0 / 29.8 / 30.0 / 32.0 with 2 x 1500 queries of 4
+// heads of 64 on 2000. Parts of fewer than 9 tiles (16 up to D = 64, whose tiles are half the work)
+// cost more in prologues and partials than they save: 2 x 300 queries of 8 heads of 64 on 2000 keys
+// 30.3 whole, 18.3 in four parts, 21.7 in eight; a 512 window 18.4 whole, 21.7 in two.
 int fwd_default_splits(const mykfa_fwd_params& p) {
     if (p.cu_seqlens_q != nullptr || p.batch <= 0 || p.max_seqlen_q <= 0) return 1;
     const int hpw = gcd_int(p.num_heads / p.num_kv_heads, 4), rows = 4 / hpw * 32, BN = p.head_dim > 128 ? 32 : 64;
@@ -460,8 +461,9 @@ int fwd_default_splits(const mykfa_fwd_params& p) {
     long long span = (long long)p.window_left + p.window_right + rows + BN;  // most keys a block sees
     if (span > p.max_seqlen_k) span = p.max_seqlen_k;
     const long long tiles = (span + BN - 1) / BN;
-    long long splits = 256 / blocks;
-    if (splits > tiles / 8) splits = tiles / 8;
+    const int least = p.head_dim <= 64 ? 16 : 9;
+    long long splits = 448 / blocks;
+    if (splits > tiles / least) splits = tiles / least;
     if (splits > 64) splits = 64;
     return splits < 2 ? 1 : (int)splits;
 }

@@ -42,7 +42,7 @@ PyObject* py_check = nullptr;     // _lib.check: raises for a status
 PyObject* py_backward = nullptr;  // flash_attn._backward_launch: the stored-dS backward's planning
 
 constexpr int kDecodeMaxQ = 16;
-constexpr int64_t kSplitMaxRows = 128 * 128;
+constexpr int64_t kSplitMaxRows = 128 * 224;
 
 // Raises MykfaError for a failed call (the message is this thread's).
 void check(int status) {

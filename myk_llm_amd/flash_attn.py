@@ -44,8 +44,8 @@ _UNBOUNDED = _lib.UNBOUNDED  # flash_attn.py:32
 _HEAD_DIMS = (16, 32, 64, 128, 256)  # flash_attn.py:322-323
 _DECODE_MAX_Q = 16  # few queries per sequence use the split-K decode kernel (flash_attn.py:364)
 # Only batches of at most this many (query, head) rows can have their keys split by the forward:
-# 128 rows a workgroup, at least two parts for each of the 256 CUs' workgroups.
-_SPLIT_MAX_ROWS = 128 * 128
+# 128 rows a workgroup, at least two parts for each of at most 448 workgroups.
+_SPLIT_MAX_ROWS = 128 * 224
 
 
 def _ds_budget_bytes() -> int:

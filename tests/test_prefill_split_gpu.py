@@ -37,7 +37,7 @@ def test_split_keys_match_oracle(nq, heads, kv_heads, d, lens, window, scale, dt
     assert_lse(lse, exp_lse)
 
 
-@pytest.mark.parametrize("sq, sk, heads", [(1024, 1024, 16), (1025, 1025, 16), (700, 1111, 8)])
+@pytest.mark.parametrize("sq, sk, heads", [(1792, 1792, 16), (1793, 1793, 16), (1024, 1024, 16), (700, 1111, 8)])
 def test_dense_batches_around_the_rule(sq, sk, heads):
     """One causal sequence on both sides of the most rows that are split, and Lq != Lk."""
     g = torch.Generator().manual_seed(sq)

@@ -114,7 +114,8 @@ __device__ inline int balanced_chunk(const DecodeArgs& a, long long K) {
     if (a.nseg <= a.batch) return 1 << 30;  // one slot per sequence: one split each
     long long A = (long long)min(a.resident, a.nseg) - a.batch;
     if (A < 1) A = a.nseg - a.batch;
-    long long T = (K + A - 1) / A;
+    // (64-bit division only where 32 bits do not hold the sum: it takes ~150 instructions.)
+    long long T = K + A < (1ll << 31) ? (long long)(((unsigned)K + (unsigned)A - 1) / (unsigned)A) : (K + A - 1) / A;
     T = (T + kTile - 1) / kTile * kTile;
     return (int)(T < kTile ? kTile : (T > (1 << 30) ? (1 << 30) : T));
 }
@@ -125,6 +126,27 @@ __device__ inline int seq_splits(int V, int T) { return V > T ? (V + T - 1) / T 
 // Keys the split holding a step's appended keys gives up to the other splits of its sequence.
 constexpr int kOwnerShort = 384;
 
+// Keys per split of a sequence of v visible keys in s splits.
+__device__ inline int split_chunk(const DecodeArgs& a, int v, int s) {
+    const int c = (v + s - 1) / s;
+    int ck = c < kTile ? kTile : (c + kTile - 1) / kTile * kTile;
+    // Splits start ck cache rows apart; power-of-two distances put concurrently
+    // starting workgroups on the same DRAM channels (measured ~15% slower).
+    if (ck > kTile && (ck & (ck - 1)) == 0) ck += kTile;
+    if (a.kn != nullptr && s > 1) {
+        // The last split also stores this step's new keys and waits for those
+        // stores before its loads: it gets kOwnerShort fewer keys than the others
+        // (as long as a tile is left), so that it does not end last (64 x 16K-cache
+        // batch, one query and the 4-query draft: 1.4-2.1 us less per layer for 160 to
+        // 512 keys, 2.1 at 384).
+        const int c2 = (v + kOwnerShort + s - 1) / s;
+        int ck2 = (c2 + kTile - 1) / kTile * kTile;
+        if (ck2 > kTile && (ck2 & (ck2 - 1)) == 0) ck2 += kTile;
+        if (v - (s - 1) * ck2 >= kTile) ck = ck2;
+    }
+    return ck;
+}
+
 struct SplitOf {
     int b;      // sequence, or -1 when the workgroup holds no split
     int split;  // index of the split within the sequence
@@ -132,6 +154,39 @@ struct SplitOf {
     int seg;    // workspace segment of split 0 (segments of a sequence are consecutive)
     int chunk;  // keys per split of the sequence (a multiple of kTile)
 };
+
+// The plan of a batch of at most 64 sequences, by each wave for itself (lane = sequence): no barrier
+// and no LDS on the way to the first loads (with the first tiles loaded beside Q: 64 sequences of up
+// to 16K keys 90.1 -> 89.2 us, one of 1531 keys 13.9 -> 13.2).
+__device__ inline SplitOf assign_split_wave(const DecodeArgs& a, int w, bool write_header) {
+    const int lane = threadIdx.x & 63;
+    const int v = lane < a.batch ? visible_keys(a, lane) : 0;
+    long long K = v;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) K += __shfl_xor(K, off);
+    const int T = balanced_chunk(a, K);
+    const int s = lane < a.batch ? seq_splits(v, T) : 0;
+    int inc = s;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(inc, off);
+        if (lane >= off) inc += y;
+    }
+    const int seg0 = inc - s;
+    if (write_header && lane == w && lane < a.batch) {
+        a.seg_hdr[2 * lane] = seg0;
+        a.seg_hdr[2 * lane + 1] = s;
+    }
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(w >= seg0 && w < inc);
+    SplitOf r = {-1, 0, 0, 0, 0};
+    if (hit == 0) return r;
+    r.b = __builtin_ctzll(hit);
+    r.n = __builtin_amdgcn_readlane(s, r.b);
+    r.seg = __builtin_amdgcn_readlane(seg0, r.b);
+    r.split = w - r.seg;
+    r.chunk = split_chunk(a, __builtin_amdgcn_readlane(v, r.b), r.n);
+    return r;
+}
 
 // Workgroup w's split of the length-balanced split-K: the sequences' visible key counts V_b
 // are read on the device (every workgroup computes the same plan), T follows from their sum
@@ -194,27 +249,11 @@ __device__ SplitOf assign_split(const DecodeArgs& a, int w, bool write_header, i
         const int seg0 = before + inc - s;
         if (b < a.batch) {
             if (w >= seg0 && w < seg0 + s) {
-                const int c = (v + s - 1) / s;
                 slot[0] = b;
                 slot[1] = w - seg0;
                 slot[2] = s;
                 slot[3] = seg0;
-                int ck = c < kTile ? kTile : (c + kTile - 1) / kTile * kTile;
-                // Splits start ck cache rows apart; power-of-two distances put concurrently
-                // starting workgroups on the same DRAM channels (measured ~15% slower).
-                if (ck > kTile && (ck & (ck - 1)) == 0) ck += kTile;
-                if (a.kn != nullptr && s > 1) {
-                    // The last split also stores this step's new keys and waits for those
-                    // stores before its loads: it gets kOwnerShort fewer keys than the others
-                    // (as long as a tile is left), so that it does not end last (64 x 16K-cache
-                    // batch, one query and the 4-query draft: 1.4-2.1 us less per layer for 160 to
-                    // 512 keys, 2.1 at 384).
-                    const int c2 = (v + kOwnerShort + s - 1) / s;
-                    int ck2 = (c2 + kTile - 1) / kTile * kTile;
-                    if (ck2 > kTile && (ck2 & (ck2 - 1)) == 0) ck2 += kTile;
-                    if (v - (s - 1) * ck2 >= kTile) ck = ck2;
-                }
-                slot[4] = ck;
+                slot[4] = split_chunk(a, v, s);
             }
             if (write_header && b == w) {
                 a.seg_hdr[2 * b] = seg0;
@@ -254,7 +293,9 @@ __global__ __launch_bounds__(kThreads) void decode_splitk_kernel(DecodeArgs a) {
     // kWaves consecutive (KV head, row tile) units z * kWaves ..; one unit per wave: the waves of
     // a workgroup read adjacent heads of the same cache rows and share nothing after the plan.
     __shared__ int plan_red[2 * kWaves + 5];
-    const SplitOf so = assign_split<kThreads>(a, blockIdx.x, blockIdx.z == 0 && a.seg_hdr != nullptr, plan_red);
+    const bool header = blockIdx.z == 0 && a.seg_hdr != nullptr;
+    const SplitOf so = a.batch <= 64 ? assign_split_wave(a, blockIdx.x, header && wave == 0)
+                                     : assign_split<kThreads>(a, blockIdx.x, header, plan_red);
     if (so.b < 0) return;
     const int split = so.split, b = so.b;
     const int unit = blockIdx.z * kWaves + wave;
@@ -266,49 +307,6 @@ __global__ __launch_bounds__(kThreads) void decode_splitk_kernel(DecodeArgs a) {
     const int k0 = rg.lo + split * so.chunk;
     const int k1 = k0 + so.chunk < rg.hi ? k0 + so.chunk : rg.hi;  // k1 <= k0 only for an empty sequence
     const int lo_off = band_lo(L, a.nq, a.wl), hi_off = band_hi(L, a.nq, a.wr);
-
-    // Q^T operand: lane holds Q[row l16][32 kk + 8 G + i]. Issued before the appended keys'
-    // loads, so that their latencies overlap (the stores wait for the new keys' data).
-    const int row = rt * 16 + l16;
-    const bool row_ok = row < a.rows;
-    const int gh = row_ok ? row / a.nq : 0, qi = row_ok ? row % a.nq : 0;
-    const int h = kvh * a.group + gh;
-    s16x8 qop[KD];
-    {
-        const uint16_t* qp = a.q + (int64_t)b * a.qbs + (int64_t)qi * a.qts + (int64_t)h * a.qhs;
-#pragma unroll
-        for (int kk = 0; kk < KD; ++kk) {
-            s16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-            const int d0 = 32 * kk + 8 * G;
-            if (row_ok && d0 < D) v = ld16(qp + d0);
-            qop[kk] = v;
-        }
-    }
-    if (a.kn) {
-        // This step's new keys first (flash_attn.py:480-485): the wave writes the rows of its KV
-        // head that fall in its split's key range (rows before the visible range go to split 0),
-        // whatever their visibility, and drops rows at or beyond the capacity. Every wave
-        // reading a row wrote it itself (waves of further row tiles of a head write identical
-        // copies), and the wait below orders its stores before its loads.
-        const int base = a.seqused_k[b];
-        constexpr int CPR = D / 8;
-        for (int i = lane; i < a.n_new * CPR; i += 64) {
-            const int t = i / CPR, ch = i % CPR;
-            const int pos = base + t;
-            const int owner = pos < rg.lo ? 0 : min((pos - rg.lo) / so.chunk, so.n - 1);
-            if (pos < 0 || pos >= a.cap || owner != split) continue;
-            const int64_t src_k = (int64_t)b * a.knbs + (int64_t)t * a.knts + (int64_t)kvh * a.knhs + ch * 8;
-            const int64_t src_v = (int64_t)b * a.vnbs + (int64_t)t * a.vnts + (int64_t)kvh * a.vnhs + ch * 8;
-            const int64_t dst_k = (int64_t)b * a.kbs + (int64_t)pos * a.kts + (int64_t)kvh * a.khs + ch * 8;
-            const int64_t dst_v = (int64_t)b * a.vbs + (int64_t)pos * a.vts + (int64_t)kvh * a.vhs + ch * 8;
-            st16(const_cast<uint16_t*>(a.k) + dst_k, ld16(a.kn + src_k));
-            st16(const_cast<uint16_t*>(a.v) + dst_v, ld16(a.vn + src_v));
-        }
-    }
-    // Q landed (and any appended rows stored) before the ring's loads share the in-order
-    // counter; otherwise the counter analysis cannot bound the loop's pending loads and drains
-    // them at the loop head.
-    wait_vmcnt<0>();
 
     // K / V rows 0 .. L-1 of this (sequence, KV head) through bounds-checked buffer loads: keys
     // at or beyond L read 0 and a load whose offset is at or above 2^31 fetches nothing, which
@@ -338,11 +336,6 @@ __global__ __launch_bounds__(kThreads) void decode_splitk_kernel(DecodeArgs a) {
         voff[i] = (unsigned)(idx / (D / 8)) * vts2 + (idx % (D / 8)) * 16;
     }
 
-    f32x4 acc[DB];
-#pragma unroll
-    for (int db = 0; db < DB; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-    float m_i = kNegFloor, l_i = 0.f;
-
     struct TileRegs {
         s16x8 k[VPL];
         s16x8 v[VPL];
@@ -360,6 +353,66 @@ __global__ __launch_bounds__(kThreads) void decode_splitk_kernel(DecodeArgs a) {
         // tile alone; a scheduler that interleaves two tiles' loads forces a full drain.
         __builtin_amdgcn_sched_barrier(0);
     };
+    // Q^T operand: lane holds Q[row l16][32 kk + 8 G + i]. Issued before the appended keys'
+    // loads, so that their latencies overlap (the stores wait for the new keys' data).
+    const int row = rt * 16 + l16;
+    const bool row_ok = row < a.rows;
+    const int gh = row_ok ? row / a.nq : 0, qi = row_ok ? row % a.nq : 0;
+    const int h = kvh * a.group + gh;
+    s16x8 qop[KD];
+    {
+        const uint16_t* qp = a.q + (int64_t)b * a.qbs + (int64_t)qi * a.qts + (int64_t)h * a.qhs;
+#pragma unroll
+        for (int kk = 0; kk < KD; ++kk) {
+            s16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+            const int d0 = 32 * kk + 8 * G;
+            if (row_ok && d0 < D) v = ld16(qp + d0);
+            qop[kk] = v;
+        }
+    }
+    // A split that stores new keys reads its tiles after that; the others' first tiles go out with
+    // Q, in one memory latency.
+    TileRegs buf[NBUF];
+    auto first_tiles = [&]() {
+#pragma unroll
+        for (int i = 0; i < NBUF - 1; ++i) load_tile(k0 + i * kTile, buf[i]);
+    };
+    const int base = a.kn ? a.seqused_k[b] : 0;
+    auto owner_of = [&](int pos) { return pos < rg.lo ? 0 : min((pos - rg.lo) / so.chunk, so.n - 1); };
+    const bool owner = a.kn && split >= owner_of(base) && split <= owner_of(base + a.n_new - 1);
+    if (!owner) first_tiles();
+    if (owner) {
+        // This step's new keys first (flash_attn.py:480-485): the wave writes the rows of its KV
+        // head that fall in its split's key range (rows before the visible range go to split 0),
+        // whatever their visibility, and drops rows at or beyond the capacity. Every wave
+        // reading a row wrote it itself (waves of further row tiles of a head write identical
+        // copies), and the wait below orders its stores before its loads.
+        constexpr int CPR = D / 8;
+        for (int i = lane; i < a.n_new * CPR; i += 64) {
+            const int t = i / CPR, ch = i % CPR;
+            const int pos = base + t;
+            if (pos < 0 || pos >= a.cap || owner_of(pos) != split) continue;
+            const int64_t src_k = (int64_t)b * a.knbs + (int64_t)t * a.knts + (int64_t)kvh * a.knhs + ch * 8;
+            const int64_t src_v = (int64_t)b * a.vnbs + (int64_t)t * a.vnts + (int64_t)kvh * a.vnhs + ch * 8;
+            const int64_t dst_k = (int64_t)b * a.kbs + (int64_t)pos * a.kts + (int64_t)kvh * a.khs + ch * 8;
+            const int64_t dst_v = (int64_t)b * a.vbs + (int64_t)pos * a.vts + (int64_t)kvh * a.vhs + ch * 8;
+            st16(const_cast<uint16_t*>(a.k) + dst_k, ld16(a.kn + src_k));
+            st16(const_cast<uint16_t*>(a.v) + dst_v, ld16(a.vn + src_v));
+        }
+    }
+    // Q and the first tiles landed before the loop (otherwise the counter analysis cannot bound the
+    // loop's pending loads and drains them at its head); appended rows stored before their reads.
+    wait_vmcnt<0>();
+    if (owner) {
+        first_tiles();
+        wait_vmcnt<0>();
+    }
+
+    f32x4 acc[DB];
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_i = kNegFloor, l_i = 0.f;
+
     auto compute_tile = [&](int t0, const TileRegs& tr, int parity) {
         // Stage K and V in this wave's LDS (swizzled rows) for the operand reads.
         uint16_t* ks = klds[wave][parity % NPAR];
@@ -437,9 +490,6 @@ __global__ __launch_bounds__(kThreads) void decode_splitk_kernel(DecodeArgs a) {
 
     // NBUF tiles in registers: tile j computes while tiles j + 1 .. j + NBUF - 1 are in flight.
     const int nt = k1 > k0 ? (k1 - k0 + kTile - 1) / kTile : 0;
-    TileRegs buf[NBUF];
-#pragma unroll
-    for (int i = 0; i < NBUF - 1; ++i) load_tile(k0 + i * kTile, buf[i]);
     for (int t = 0; t < nt; t += NBUF) {
 #pragma unroll
         for (int i = 0; i < NBUF; ++i) {

@@ -508,6 +508,33 @@ struct Plan {
     Size size;
     int splits;
 };
+// Stages of the product that one more part of every result costs in fp32 partials written and read
+// back (256 x 256 x 8 bytes at the copy rate against 1.6 us a stage, both over the whole chip).
+constexpr double kPartStages = 19;
+
+// Rounds of the CUs that `units` of the 256 x 256 tiles take; a short last round runs as quarters.
+double big_rounds(long long units) {
+    const long long rest = units % kCUs;
+    return (double)(units / kCUs) + (rest == 0 ? 0. : units > kCUs && rest <= kCUs / 2 ? .85 : 1.);
+}
+// Parts of K for the 256 x 256 tiles that take the least time, over up to three rounds. With one
+// round only, tiles just above a half or a third of the CUs went to the 128 x 128 tile whole: rows x
+// 1024 x 65536 with 10000 rows (160 tiles, now in 3 parts) 1996 -> 1260 us, 5632 (88, 8) 957 -> 728, 6144
+// (96, 8) 869 -> 811; counts that divide the CUs evenly as they were.
+int big_splits(long long tiles, int stages) {
+    int best = 1;
+    double least = 0;
+    for (int s = 1; s == 1 || (s <= stages / 16 && tiles * s <= 3 * kCUs); ++s) {
+        const int per = (stages + s - 1) / s;
+        if (s > 1 && (stages + per - 1) / per != s) continue;  // every split holds a stage
+        const double cost = big_rounds(tiles * s) * kCUs * per / tiles + (s > 1 ? kPartStages * s : 0);
+        if (s == 1 || cost < least) {
+            best = s;
+            least = cost;
+        }
+    }
+    return best;
+}
 // K is split only for bf16 results without an addend, into at least 16 stages each.
 Plan plan_of(const mykfa_gemm_params& p) {
     const int stages = (p.k + kBK - 1) / kBK;
@@ -515,7 +542,9 @@ Plan plan_of(const mykfa_gemm_params& p) {
     for (int size = BIG; size <= SMALL; ++size) {
         const long long tiles = tile_count(p.m, p.n, p.batch, 256 >> size);
         int splits = 1;
-        if (can_split && tiles <= kCUs / 2) {
+        if (can_split && size == BIG) {
+            splits = big_splits(tiles, stages);
+        } else if (can_split && tiles <= kCUs / 2) {
             splits = (int)(kCUs / tiles);
             if (splits > stages / 16) splits = stages / 16;
             if (splits < 1) splits = 1;

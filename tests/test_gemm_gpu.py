@@ -28,7 +28,8 @@ def _close(got, exp, k, bf16):
 
 @pytest.mark.parametrize("b, m, n, k", [
     (1, 1, 8, 8), (1, 64, 64, 64), (3, 65, 72, 63), (2, 129, 200, 129), (9, 257, 264, 328), (1, 1000, 2056, 72),
-    (1, 2048, 16640, 192), (1, 256, 512, 4104), (2, 127, 130, 2000), (1, 300, 33, 8200), (7, 1024, 2048, 320)])
+    (1, 2048, 16640, 192), (1, 256, 512, 4104), (2, 127, 130, 2000), (1, 300, 33, 8200), (7, 1024, 2048, 320),
+    (1, 2500, 4000, 8200), (1, 2500, 7600, 8200)])  # K parts over two rounds, and a last round in quarters
 def test_products_match_float64(b, m, n, k):
     print(f"gemm {b} x {m} x {n} x {k}", flush=True)
     g = torch.Generator().manual_seed(m + n + k)

@@ -15,9 +15,9 @@ gradient is computed during the forward pass, so the loss is backpropagated exac
 
 The products are libmykfa.so's (csrc/gemm.hip) where the hidden size is a multiple of 8, else
 torch.matmul's. The weight gradient accumulates in fp32 inside its product instead of rounding each
-chunk's bf16 product before an fp32 add (fused_ce.py:89), and takes the tokens of several chunks at
-once: the chunks' d logits are kept in a buffer of up to _KEEP_BYTES (one chunk where that, or the
-device's memory, holds no more).
+chunk's bf16 product before an fp32 add (fused_ce.py:89). A chunk there holds as many tokens as
+_KEEP_BYTES of d logits do, in even passes over the tokens, and chunk_size at least (chunk_size where
+the device's memory holds no more).
 """
 
 from __future__ import annotations
@@ -54,11 +54,13 @@ def _chunk_spans(n: int, size: int) -> list[tuple[int, int]]:
     return [(lo, min(lo + size, n)) for lo in range(0, n, size)]
 
 
-# d logits kept for one weight-gradient product. Its fp32 sums are read and written once per
-# product: 65536 x 1024 over 8192 tokens takes 4 x 335 us in chunks of 2048 with the sums read back,
-# 990 at once; the whole head over 16384 tokens 8137 us with one chunk kept, 7746, 7599 and 7506 with
-# two, four and eight.
-_KEEP_BYTES = 1 << 30
+# d logits in memory at once. One pass's products run over all its tokens: fewer rounds of workgroups
+# cut short, fewer fp32 partials of d hidden, and the fp32 d weight is read and written once per pass
+# (65536 x 1024 over 8192 tokens 990 us at once, 4 x 335 in chunks of 2048). Whole head, chunks of 2048
+# with up to 1 GiB kept for d weight alone, against passes of up to this: 16384 tokens of hidden 1024 and
+# vocabulary 65536 7280 -> 7000 us (1.5 GiB the same, 1 GiB 7370: three passes), 32000 3510 -> 3365; 512 and 8000
+# 836 -> 638; 3000 tokens of 1024 and 32000 750 -> 725.
+_KEEP_BYTES = 5 << 28
 
 
 def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: float, z_coef: float,
@@ -87,20 +89,26 @@ def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: 
         h16, w16 = (x if usable(x) else x.contiguous() for x in (h16, w16))
         d_weight = torch.empty((vocab, width), dtype=torch.float32, device=dev)
         chunk = min(chunk_size, tokens)
-        kept = max(1, min(_KEEP_BYTES // (2 * chunk * stride), (tokens + chunk - 1) // chunk)) * chunk
+        passes = -(-tokens // max(chunk, _KEEP_BYTES // (2 * stride)))
+        rows = min(tokens, (-(-tokens // passes) + 255) // 256 * 256)
+
+        def run(rows: int) -> None:
+            blocks = torch.empty((rows, stride), dtype=torch.bfloat16, device=dev)
+            for lo, hi in _chunk_spans(tokens, rows):
+                block, h = blocks[:hi - lo, :vocab], h16[lo:hi]
+                gemm(h, w16, block, hi - lo, vocab, width, b_transposed=True)
+                _ce_rows(block, tgt[lo:hi], row_stats[0, lo:hi], row_stats[1, lo:hi], scale, z_coef, ignore_index)
+                gemm(block, w16, d_hidden[lo:hi], hi - lo, width, vocab)
+                gemm(block, h, d_weight, vocab, width, hi - lo, a_transposed=True, beta=0.0 if lo == 0 else 1.0)
+
         try:
-            blocks = torch.empty((kept, stride), dtype=torch.bfloat16, device=dev)
+            run(rows)
         except torch.OutOfMemoryError:
-            kept = chunk
-            blocks = torch.empty((kept, stride), dtype=torch.bfloat16, device=dev)
-        for first, last in _chunk_spans(tokens, kept):
-            for lo, hi in _chunk_spans(last - first, chunk):
-                block, a, b = blocks[lo:hi, :vocab], first + lo, first + hi
-                gemm(h16[a:b], w16, block, b - a, vocab, width, b_transposed=True)
-                _ce_rows(block, tgt[a:b], row_stats[0, a:b], row_stats[1, a:b], scale, z_coef, ignore_index)
-                gemm(block, w16, d_hidden[a:b], b - a, width, vocab)
-            gemm(blocks, h16[first:last], d_weight, vocab, width, last - first, a_transposed=True,
-                 beta=0.0 if first == 0 else 1.0)
+            if rows <= chunk:
+                raise
+            rows = 0
+        if rows == 0:  # past the handler, which holds the larger buffer
+            run(chunk)
         return row_stats, d_hidden, d_weight
     d_weight = torch.zeros(weight.shape, dtype=torch.float32, device=dev)
     for lo, hi in _chunk_spans(tokens, chunk_size):

@@ -209,8 +209,18 @@ def test_rows_with_a_vocabulary_tail(rows, vocab, stride, dtype):
 @pytest.mark.parametrize("tokens, width, vocab, chunk, keep", [(100, 72, 1003, 33, 1 << 30), (100, 72, 1003, 33, 1), (517, 64, 264, 128, 2 * 264 * 2 * 128)])
 @pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)])
 def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, dtypes):
-    """Any number of chunks per weight-gradient product gives the reference's loss and gradients."""
+    """Any number of passes gives the reference's loss and gradients; one pass too large for the
+    device's memory is taken back for passes of chunk_size."""
     monkeypatch.setattr(fused_ce, "_KEEP_BYTES", keep)
+    real, refused = fused_ce.gemm, []
+
+    def scarce(a, b, c, m, n, k, **kw):
+        if kw.get("a_transposed") and k > chunk and tokens > 500:  # no memory for the larger passes
+            refused.append(k)
+            raise torch.OutOfMemoryError("planted")
+        real(a, b, c, m, n, k, **kw)
+
+    monkeypatch.setattr(fused_ce, "gemm", scarce)
     g = torch.Generator().manual_seed(tokens)
     hidden = torch.randn(tokens, width, generator=g).to(torch.bfloat16).to(dtypes[0]).cuda().requires_grad_()
     weight = (0.1 * torch.randn(vocab, width, generator=g)).to(torch.bfloat16).to(dtypes[1]).cuda().requires_grad_()
@@ -219,6 +229,7 @@ def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, 
     n = float((targets != -100).sum())
     loss, ce_sum, z_sum = fused_ce.fused_linear_cross_entropy(hidden, weight, targets, n, 1e-3, chunk_size=chunk)
     (3.0 * loss).backward()
+    assert len(refused) == (tokens > 500)
     h, w = (x.detach().double().requires_grad_() for x in (hidden, weight))
     logits = h @ w.t()
     lse = torch.logsumexp(logits, -1)

@@ -28,14 +28,15 @@
 // Bound by the matrix cores at the clock that the card holds under this load (~1.9 GHz: MFMA busy
 // 62 % at 8192 x 8192 x 8192, LDS active 24 %); zeros for data run 35 % faster.
 #include "common.h"
+#include "gemm_tiles.h"
 #include "kernels.h"
 
 namespace mykfa {
 namespace {
 
-constexpr int kBK = 64;            // K columns per stage
+constexpr int kBK = kGemmBK;
 constexpr int kKS = kBK / 16;      // k-steps per stage
-constexpr int kCUs = 256;
+constexpr int kCUs = kGemmCUs;
 constexpr unsigned kSkip = 0x80000000u;  // an offset outside any buffer: the load returns zero
 
 struct GemmArgs {
@@ -48,11 +49,9 @@ struct GemmArgs {
     int64_t c_bs, c_rs, d_bs, d_rs;
     float alpha, beta;
     bool c_vec, d_vec;  // 16-byte rows of C / Add (else 8-byte / 2-byte accesses; SYM only)
-    int batch, splits;
-    // A launch that takes the last units of a larger tile's list, each as four quarters.
-    int first_unit;
-    bool quarters;
-    int tm, tn, stages, per_xcd, units;  // set by launch(): stages per split; units of this launch
+    int batch;
+    GemmGrid g;
+    int per_xcd, units;  // of this launch
 };
 
 enum Out { OUT_BF16, OUT_ADD, OUT_F32, OUT_PART, OUT_SYM };  // OUT_BF16: no addend
@@ -67,7 +66,7 @@ struct Operand {
     unsigned voff[LOADS];  // of this wave's loads, the same for every tile
     int64_t rs;
     uint64_t base;
-    int rows, cols;  // stored rows and columns from the tile's origin
+    GemmPart part;
 
     __device__ inline void offsets(int64_t rstride, int wave, int lane) {
         rs = rstride;
@@ -80,27 +79,16 @@ struct Operand {
     }
     // The tile whose first row (column) of `mn` is r0.
     __device__ inline void enter(const uint16_t* p, int mn, int k, int r0) {
-        if constexpr (TR) {
-            base = reinterpret_cast<uint64_t>(p + r0);
-            rows = k;
-            cols = ((mn + 7) & ~7) - r0;
-        } else {
-            base = reinterpret_cast<uint64_t>(p + (int64_t)r0 * rs);
-            rows = max(min(mn - r0, R), 0);  // none: a quarter past the edge
-            cols = (k + 7) & ~7;
-        }
+        part = gemm_part<TR>(mn, k, r0, R);
+        base = reinterpret_cast<uint64_t>(p + (int64_t)part.row0 * rs + part.col0);
     }
     // This wave's loads of K stage kt into the tile at LDS address lds. Rows past the matrix read
     // zero through the descriptor; chunks past K through their offset.
     __device__ inline void issue(int kt, uint32_t lds, int wave, int lane) const {
-        const int k0 = kt * kBK;
-        i32x4 rsrc;
-        if constexpr (TR) {
-            const int r = rows - k0 < kBK ? rows - k0 : kBK;
-            rsrc = buffer_rsrc32(base + (uint64_t)k0 * (uint64_t)(rs * 2), r > 0 ? ((r - 1) * (int)rs + cols) * 2 : 0);
-        } else {
-            const int left = cols - k0;
-            rsrc = buffer_rsrc32(base + (uint64_t)(unsigned)(k0 * 2), left > 0 && rows > 0 ? ((rows - 1) * (int)rs + left) * 2 : 0);
+        const GemmSpan s = gemm_span<TR>(part, (int)rs, kt);
+        const i32x4 rsrc = buffer_rsrc32(base + ((uint64_t)(unsigned)s.row * (uint64_t)rs + (unsigned)s.col) * 2, s.bytes);
+        if constexpr (!TR) {
+            const int left = part.cols - s.col;
             if (left < kBK) {
 #pragma unroll
                 for (int j = 0; j < LOADS; ++j) {
@@ -155,10 +143,6 @@ __device__ inline s16x8 load8(const uint16_t* d, int left, bool vec) {
     return w;
 }
 
-struct Tile {
-    int outer, bidx, m0, n0, kt0, nk;  // outer = batch * splits + split; K stages [kt0, kt0 + nk)
-};
-
 template <int WM, int WN, int MI, int NI, int STAGES, int OCC, bool AT, bool BT, int OUT>
 __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
     constexpr int NW = WM * WN, BM = WM * MI * 32, BN = WN * NI * 32;
@@ -179,30 +163,17 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
     const int end = min((xcd + 1) * p.per_xcd, p.units);
     const int first = xcd * p.per_xcd + (int)(blockIdx.x / kXcds);
     if (first >= end) return;
-    // Unit -> (batch, split, tile). Groups of up to 8 row tiles run down the columns (SYM: row by
-    // row of the lower triangle), so the tiles resident on an XCD share its L2's panels.
+    // Unit -> (batch, split, tile); SYM: row by row of the lower triangle.
     auto tile_of = [&](int unit) {
-        Tile t;
-        const int quad = p.quarters ? unit & 3 : 0, side = p.quarters ? 2 : 1;
-        unit = p.first_unit + (p.quarters ? unit >> 2 : unit);
-        const int tiles = OUT == OUT_SYM ? p.tm * (p.tm + 1) / 2 : p.tm * p.tn;
-        t.outer = unit / tiles;
-        const int x = unit % tiles;
-        t.bidx = t.outer / p.splits;
-        t.kt0 = t.outer % p.splits * p.stages;
-        t.nk = min(p.stages, max((p.k + kBK - 1) / kBK, 1) - t.kt0);
         if constexpr (OUT == OUT_SYM) {
+            const int tiles = p.g.tm * (p.g.tm + 1) / 2, x = unit % tiles, bidx = unit / tiles;
             int r = (int)((sqrtf(8.0f * (float)x + 1.0f) - 1.0f) * 0.5f);
             while (r * (r + 1) / 2 > x) --r;
             while ((r + 1) * (r + 2) / 2 <= x) ++r;
-            t.m0 = r * BM;
-            t.n0 = (x - r * (r + 1) / 2) * BN;
+            return GemmTile{bidx, bidx, r * BM, (x - r * (r + 1) / 2) * BN, 0, p.g.stages};
         } else {
-            const int gsz = 8 * p.tn, grp = x / gsz, in = x % gsz, gm = min(8, p.tm - grp * 8);
-            t.m0 = ((grp * 8 + in % gm) * side + (quad & 1)) * BM;
-            t.n0 = (in / gm * side + (quad >> 1)) * BN;
+            return gemm_tile(p.g, p.k, unit, BM, BN);
         }
-        return t;
     };
 
     // The loads run ahead of the products: stage lk of unit lu (tile lt) goes to slot lslot next;
@@ -212,7 +183,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
     oa.offsets(p.a_rs, wave, lane);
     ob.offsets(p.b_rs, wave, lane);
     int lu = first, lk = 0, lslot = 0, ahead = 0;
-    Tile lt = tile_of(lu);
+    GemmTile lt = tile_of(lu);
     auto enter = [&]() {
         oa.enter(p.a + lt.bidx * p.a_bs, p.m, p.k, lt.m0);
         ob.enter(p.b + lt.bidx * p.b_bs, p.n, p.k, lt.n0);
@@ -274,7 +245,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
     read(0, 0);
 
     for (int unit = first; unit < end; unit += step) {
-        const Tile t = tile_of(unit);
+        const GemmTile t = tile_of(unit);
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -478,11 +449,11 @@ long long tile_count(int m, int n, int batch, int t) {
 template <bool AT, bool BT, int OUT>
 hipError_t launch_size(GemmArgs a, Size size, hipStream_t s) {
     const int side = 256 >> size;
-    a.tm = (a.m + side - 1) / side;
-    a.tn = (a.n + side - 1) / side;
-    const int all = a.k > 0 ? (a.k + kBK - 1) / kBK : 1;
-    a.stages = (all + a.splits - 1) / a.splits;
-    const long long units = (OUT == OUT_SYM ? (long long)a.tm * (a.tm + 1) / 2 : (long long)a.tm * a.tn) * a.batch * a.splits;
+    a.g.tm = (a.m + side - 1) / side;
+    a.g.tn = (a.n + side - 1) / side;
+    a.g.stages = (gemm_stages(a.k) + a.g.splits - 1) / a.g.splits;
+    const long long units =
+        (OUT == OUT_SYM ? (long long)a.g.tm * (a.g.tm + 1) / 2 : (long long)a.g.tm * a.g.tn) * a.batch * a.g.splits;
     if (units > (1ll << 30)) return hipErrorInvalidValue;
     a.units = (int)units;
     if (size == SMALL) return launch<2, 1, 1, 2, 4, 1, AT, BT, OUT>(a, s);
@@ -494,8 +465,8 @@ hipError_t launch_size(GemmArgs a, Size size, hipStream_t s) {
         a.units -= rest;
         const hipError_t e = launch<2, 4, 4, 2, 2, 2, AT, BT, OUT>(a, s);
         if (e != hipSuccess) return e;
-        a.first_unit = a.units;
-        a.quarters = true;
+        a.g.first_unit = a.units;
+        a.g.quarters = true;
         a.units = 4 * rest;
         return launch<2, 2, 2, 2, 2, 2, AT, BT, OUT>(a, s);
     }
@@ -584,13 +555,13 @@ hipError_t launch_gemm(const mykfa_gemm_params& p, void* ws, hipStream_t stream)
         };
         a.c_vec = vec(p.c, a.c_bs, a.c_rs);
         a.d_vec = vec(p.add, a.d_bs, a.d_rs);
-        a.splits = 1;
+        a.g.splits = 1;
         const long long t = (p.m + 127) / 128;
         return launch_size<false, false, OUT_SYM>(a, p.batch * (t * (t + 1) / 2) >= kCUs * 3 / 4 ? MID : SMALL, stream);
     }
     a.c_vec = a.d_vec = true;
     const Plan plan = plan_of(p);
-    a.splits = plan.splits;
+    a.g.splits = plan.splits;
     if (p.c_dtype == MYKFA_FP32) return launch_size<true, true, OUT_F32>(a, plan.size, stream);
     if (plan.splits > 1) {
         const int n8 = (p.n + 7) / 8;

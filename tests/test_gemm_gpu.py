@@ -84,3 +84,21 @@ def test_newton_schulz_odd_shapes(shape, steps, transposed):
     exp = torch.stack([om.newton_schulz_reference(m, steps) for m in x.float()])
     err = (got.float().cpu() - exp).norm() / exp.norm()
     assert err <= 2.0 ** -9 * 3.45 * steps * 2, err
+
+
+@pytest.mark.parametrize("m, n, k", [(50257, 1024, 65), (4136, 4096, 129), (4096, 4136, 1)])
+def test_quarters_past_an_edge(m, n, k):
+    """The last units of a product run as quarters, some of which begin past M or N, with one row of K in
+    the last stage: they store nothing, and the others' results are whole."""
+    print(f"quarters past an edge {m} x {n} x {k}", flush=True)
+    g = torch.Generator().manual_seed(m + k)
+    a, w = _padded(g, 1, k, m), _padded(g, 1, k, n)
+    c = torch.full((1, m, (n + 7) // 8 * 8), float("nan"), device="cuda")
+    gemm(a, w, c, m, n, k, a_transposed=True)
+    _close(c[..., :n], a[..., :m].double().transpose(1, 2).contiguous() @ w[..., :n].double(), k, False)
+    b = torch.full_like(c, float("nan"), dtype=torch.bfloat16)
+    rows = a[..., :m].transpose(1, 2).contiguous()
+    x = torch.zeros(1, m, (k + 7) // 8 * 8, dtype=torch.bfloat16, device="cuda")
+    x[..., :k] = rows
+    gemm(x, w, b, m, n, k)
+    _close(b[..., :n], rows.double() @ w[..., :n].double(), k, True)

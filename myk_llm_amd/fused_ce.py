@@ -84,7 +84,9 @@ def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: 
     # of two apart fall on few channels (2048 x 65536 x 1024 in / out: logits 291 -> 268 us, d hidden
     # 265 -> 251; rows off the lines 325 and 276).
     stride = ((vocab + 127) // 128 | 1) * 128
-    if width % 8 == 0 and width > 0 and vocab > 0 and tokens > 0 and max(stride, width) < 1 << 22:
+    # (A weight of another width is left to torch.mm, which refuses it: mykfa_gemm takes the sizes it is told.)
+    if (width % 8 == 0 and width > 0 and vocab > 0 and tokens > 0 and max(stride, width) < 1 << 22
+            and tuple(weight.shape) == (vocab, width)):
         h16 = hidden if hidden.dtype == torch.bfloat16 else hidden.to(torch.bfloat16)
         h16, w16 = (x if usable(x) else x.contiguous() for x in (h16, w16))
         d_weight = torch.empty((vocab, width), dtype=torch.float32, device=dev)

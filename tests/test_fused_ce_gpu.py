@@ -244,3 +244,11 @@ def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, 
         assert got.dtype in dtypes
         err = (got.double() - want).norm() / want.norm()
         assert err < 1e-2, err  # bf16 logits and gradients: 2^-8 each
+
+
+@pytest.mark.parametrize("shape", [(1000, 1024), (1000, 256), (1000, 512, 1), (512,)])
+def test_weight_of_another_width_is_refused(shape):
+    hidden = torch.randn(40, 512, dtype=torch.bfloat16, device="cuda")
+    weight = torch.randn(*shape, dtype=torch.bfloat16, device="cuda")
+    with pytest.raises(RuntimeError, match="shape|size|dim|2D|matri"):
+        fused_linear_cross_entropy(hidden, weight, torch.zeros(40, dtype=torch.int64, device="cuda"), 40.0)

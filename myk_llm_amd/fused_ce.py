@@ -88,7 +88,10 @@ def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: 
     if (width % 8 == 0 and width > 0 and vocab > 0 and tokens > 0 and max(stride, width) < 1 << 22
             and tuple(weight.shape) == (vocab, width)):
         h16 = hidden if hidden.dtype == torch.bfloat16 else hidden.to(torch.bfloat16)
-        h16, w16 = (x if usable(x) else x.contiguous() for x in (h16, w16))
+        # Rows at most 2^22 apart (a tile's 256 within 2 GiB). A clone and not contiguous(), which hands back a
+        # contiguous tensor that starts off 16 bytes, or a single row of an odd stride, as it is.
+        h16, w16 = (x if usable(x) and x.stride(0) <= 1 << 22 else x.clone(memory_format=torch.contiguous_format)
+                    for x in (h16, w16))
         d_weight = torch.empty((vocab, width), dtype=torch.float32, device=dev)
         chunk = min(chunk_size, tokens)
         passes = -(-tokens // max(chunk, _KEEP_BYTES // (2 * stride)))

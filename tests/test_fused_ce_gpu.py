@@ -252,3 +252,33 @@ def test_weight_of_another_width_is_refused(shape):
     weight = torch.randn(*shape, dtype=torch.bfloat16, device="cuda")
     with pytest.raises(RuntimeError, match="shape|size|dim|2D|matri"):
         fused_linear_cross_entropy(hidden, weight, torch.zeros(40, dtype=torch.int64, device="cuda"), 40.0)
+
+
+def _flat_view(x, offset):
+    """x's values in a view that starts `offset` elements into a flat buffer."""
+    flat = torch.zeros(offset + x.numel(), dtype=x.dtype, device=x.device)
+    return flat[offset:].view(x.shape).copy_(x)
+
+
+def _far_rows(x):
+    """x's rows so far apart that a tile of 256 spans more than 2 GiB."""
+    step = (1 << 22) + (1 << 15)
+    return torch.empty(step * (x.shape[0] - 1) + x.shape[1], dtype=x.dtype, device=x.device).as_strided(x.shape, (step, 1)).copy_(x)
+
+
+@pytest.mark.parametrize("tokens, hidden_as, weight_as", [
+    (30, lambda x: x, lambda w: _flat_view(w, 1)), (30, lambda x: _flat_view(x, 3), lambda w: w),
+    (1, lambda x: x.new_zeros(1, 65).as_strided((1, 64), (65, 1)).copy_(x), lambda w: w), (30, _far_rows, lambda w: w),
+    (30, lambda x: x.t().contiguous().t(), lambda w: w.t().contiguous().t())])
+def test_layouts_that_the_products_do_not_read(tokens, hidden_as, weight_as):
+    """The same bits as for plain tensors: such layouts are copied, not refused."""
+    g = torch.Generator().manual_seed(tokens)
+    hidden = torch.randn(tokens, 64, generator=g).to(torch.bfloat16).cuda()
+    weight = (0.1 * torch.randn(300, 64, generator=g)).to(torch.bfloat16).cuda()
+    targets = torch.randint(0, 300, (tokens,), generator=g).cuda()
+    results = []
+    for h, w in ((hidden, weight), (hidden_as(hidden), weight_as(weight))):
+        h, w = h.detach().requires_grad_(), w.detach().requires_grad_()
+        loss, ce_sum, z_sum = fused_linear_cross_entropy(h, w, targets, float(tokens), 1e-3)
+        results.append((loss, ce_sum, z_sum, *torch.autograd.grad(loss, (h, w))))
+    assert all(torch.equal(a, b) for a, b in zip(*results))

@@ -156,7 +156,8 @@ __device__ inline void store_chunk(uint16_t* base, int c, int vocab, s16x8 v) {
 template <typename T, int VPT, bool TAIL>
 __global__ __launch_bounds__(kCeThreads) void ce_rows_resident_kernel(mykfa_ce_params p) {
     constexpr int NC = VPT / 8;  // 16-byte chunks per lane
-    constexpr bool kKeepP = T::code == MYKFA_BF16;
+    // (Rows with a tail recompute every exponential, as the streaming kernel that ran them did.)
+    constexpr bool kKeepP = T::code == MYKFA_BF16 && !TAIL;
     __shared__ float red[kCeWaves];
     const int64_t row = blockIdx.x;
     uint16_t* base = static_cast<uint16_t*>(p.logits) + row * p.row_stride;

@@ -282,3 +282,23 @@ def test_layouts_that_the_products_do_not_read(tokens, hidden_as, weight_as):
         loss, ce_sum, z_sum = fused_linear_cross_entropy(h, w, targets, float(tokens), 1e-3)
         results.append((loss, ce_sum, z_sum, *torch.autograd.grad(loss, (h, w))))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("rows, vocab", [(7, 1003), (5, 32003), (3, 65535)])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_gradients_of_a_vocabulary_tail_are_rounded_once(rows, vocab, aligned):
+    """Rows whose vocabulary 8 does not divide, padded to aligned rows or not: the gradient off the target
+    column is the fp32 value rounded once, half a bf16 ulp and the fp32 error itself, which is the exponent's:
+    |x - lse| log2(e) below 64 in fp32 and the sum of the row, together below 2^-17 of the value (2^-9 ulp)."""
+    g = torch.Generator().manual_seed(vocab)
+    x = (3 * torch.randn(rows, vocab, generator=g)).to(torch.bfloat16)
+    stride = (vocab + 7) // 8 * 8 if aligned else vocab
+    logits = torch.empty(rows, stride, dtype=torch.bfloat16, device="cuda")[:, :vocab].copy_(x)
+    targets = torch.randint(0, vocab, (rows,), generator=g)
+    ce, lse = torch.empty(rows, device="cuda"), torch.empty(rows, device="cuda")
+    _ce_rows(logits, targets.cuda(), ce, lse, 1.0 / 7, 1e-3, -100)
+    ref = torch.tensor(oc.ce_rows(x.double().numpy(), targets.numpy(), 1.0 / 7, 1e-3)[0])
+    err = (logits.cpu().double() - ref).abs() / storage_ulp(ref, torch.bfloat16).double()
+    err[torch.arange(rows), targets] = 0
+    _say(f"rows of {vocab}, aligned {aligned}: {err.max().item():.4f} ulp")
+    assert err.max() <= 0.5 + 2.0 ** -9

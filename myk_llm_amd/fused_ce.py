@@ -63,6 +63,14 @@ def _chunk_spans(n: int, size: int) -> list[tuple[int, int]]:
 _KEEP_BYTES = 5 << 28
 
 
+def _pass_rows(tokens: int, row_bytes: int, chunk_size: int) -> int:
+    """Tokens per pass: even passes over all of them, whole 256-row tiles where that fits, of at most
+    _KEEP_BYTES of d logits or chunk_size tokens, whichever is more."""
+    most = max(chunk_size, _KEEP_BYTES // row_bytes)
+    passes = -(-tokens // most)
+    return min(tokens, most, (-(-tokens // passes) + 255) // 256 * 256)
+
+
 def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: float, z_coef: float,
                         ignore_index: int, chunk_size: int) -> tuple[Tensor, Tensor, Tensor]:
     """One pass over the tokens in chunks. Returns (row_stats, d_hidden, d_weight):
@@ -94,8 +102,7 @@ def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: 
                     for x in (h16, w16))
         d_weight = torch.empty((vocab, width), dtype=torch.float32, device=dev)
         chunk = min(chunk_size, tokens)
-        passes = -(-tokens // max(chunk, _KEEP_BYTES // (2 * stride)))
-        rows = min(tokens, (-(-tokens // passes) + 255) // 256 * 256)
+        rows = _pass_rows(tokens, 2 * stride, chunk)
 
         def run(rows: int) -> None:
             blocks = torch.empty((rows, stride), dtype=torch.bfloat16, device=dev)

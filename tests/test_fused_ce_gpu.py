@@ -209,15 +209,17 @@ def test_rows_with_a_vocabulary_tail(rows, vocab, stride, dtype):
 @pytest.mark.parametrize("tokens, width, vocab, chunk, keep", [(100, 72, 1003, 33, 1 << 30), (100, 72, 1003, 33, 1), (517, 64, 264, 128, 2 * 264 * 2 * 128)])
 @pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)])
 def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, dtypes):
-    """Any number of passes gives the reference's loss and gradients; one pass too large for the
-    device's memory is taken back for passes of chunk_size."""
+    """One pass and several, the last one shorter, give the reference's loss and gradients; passes too
+    large for the device's memory are taken back for passes of chunk_size."""
     monkeypatch.setattr(fused_ce, "_KEEP_BYTES", keep)
-    real, refused = fused_ce.gemm, []
+    real, refused, passes = fused_ce.gemm, [], []
 
     def scarce(a, b, c, m, n, k, **kw):
         if kw.get("a_transposed") and k > chunk and tokens > 500:  # no memory for the larger passes
             refused.append(k)
             raise torch.OutOfMemoryError("planted")
+        if kw.get("a_transposed"):
+            passes.append(k)
         real(a, b, c, m, n, k, **kw)
 
     monkeypatch.setattr(fused_ce, "gemm", scarce)
@@ -229,7 +231,8 @@ def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, 
     n = float((targets != -100).sum())
     loss, ce_sum, z_sum = fused_ce.fused_linear_cross_entropy(hidden, weight, targets, n, 1e-3, chunk_size=chunk)
     (3.0 * loss).backward()
-    assert len(refused) == (tokens > 500)
+    assert refused == ([176] if tokens > 500 else [])
+    assert passes == ([128] * 4 + [5] if tokens > 500 else [100] if keep > 1 else [33, 33, 33, 1])
     h, w = (x.detach().double().requires_grad_() for x in (hidden, weight))
     logits = h @ w.t()
     lse = torch.logsumexp(logits, -1)

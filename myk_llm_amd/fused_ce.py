@@ -15,9 +15,8 @@ gradient is computed during the forward pass, so the loss is backpropagated exac
 
 The products are libmykfa.so's (csrc/gemm.hip) where the hidden size is a multiple of 8, else
 torch.matmul's. The weight gradient accumulates in fp32 inside its product instead of rounding each
-chunk's bf16 product before an fp32 add (fused_ce.py:89). A chunk there holds as many tokens as
-_KEEP_BYTES of d logits do, in even passes over the tokens, and chunk_size at least (chunk_size where
-the device's memory holds no more).
+chunk's bf16 product before an fp32 add (fused_ce.py:89). Without a chunk_size a pass there holds as many
+tokens as _KEEP_BYTES of d logits do (the default's 2048 where the device's memory holds no more).
 """
 
 from __future__ import annotations
@@ -63,12 +62,31 @@ def _chunk_spans(n: int, size: int) -> list[tuple[int, int]]:
 _KEEP_BYTES = 5 << 28
 
 
+class _Unset(int):
+    """chunk_size's default: its value in a signature, and not a caller's wish."""
+
+
+_CHUNK = _Unset(2048)
+
+
 def _pass_rows(tokens: int, row_bytes: int, chunk_size: int) -> int:
-    """Tokens per pass: even passes over all of them, whole 256-row tiles where that fits, of at most
-    _KEEP_BYTES of d logits or chunk_size tokens, whichever is more."""
+    """Tokens per pass: chunk_size where the caller gave one, which bounds the memory of its d logits. Else
+    even passes over all of them, whole 256-row tiles where that fits, of at most _KEEP_BYTES of d logits or
+    the default's tokens, whichever is more."""
+    if not isinstance(chunk_size, _Unset):
+        return min(chunk_size, tokens)
     most = max(chunk_size, _KEEP_BYTES // row_bytes)
     passes = -(-tokens // most)
     return min(tokens, most, (-(-tokens // passes) + 255) // 256 * 256)
+
+
+def _operand(x: Tensor) -> Tensor:
+    """x in bf16 rows that the products read, at most 2^22 elements apart (a tile's 256 within 2 GiB). A clone
+    and not contiguous(), which hands back a contiguous tensor that starts off 16 bytes, or a single row of
+    an odd stride, as it is."""
+    if x.dtype != torch.bfloat16:
+        x = x.to(torch.bfloat16)
+    return x if usable(x) and x.stride(0) <= 1 << 22 else x.clone(memory_format=torch.contiguous_format)
 
 
 def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: float, z_coef: float,
@@ -95,19 +113,15 @@ def _loss_and_gradients(hidden: Tensor, weight: Tensor, targets: Tensor, scale: 
     # (A weight of another width is left to torch.mm, which refuses it: mykfa_gemm takes the sizes it is told.)
     if (width % 8 == 0 and width > 0 and vocab > 0 and tokens > 0 and max(stride, width) < 1 << 22
             and tuple(weight.shape) == (vocab, width)):
-        h16 = hidden if hidden.dtype == torch.bfloat16 else hidden.to(torch.bfloat16)
-        # Rows at most 2^22 apart (a tile's 256 within 2 GiB). A clone and not contiguous(), which hands back a
-        # contiguous tensor that starts off 16 bytes, or a single row of an odd stride, as it is.
-        h16, w16 = (x if usable(x) and x.stride(0) <= 1 << 22 else x.clone(memory_format=torch.contiguous_format)
-                    for x in (h16, w16))
+        w16 = _operand(w16)
         d_weight = torch.empty((vocab, width), dtype=torch.float32, device=dev)
         chunk = min(chunk_size, tokens)
-        rows = _pass_rows(tokens, 2 * stride, chunk)
+        rows = _pass_rows(tokens, 2 * stride, chunk_size)
 
         def run(rows: int) -> None:
             blocks = torch.empty((rows, stride), dtype=torch.bfloat16, device=dev)
             for lo, hi in _chunk_spans(tokens, rows):
-                block, h = blocks[:hi - lo, :vocab], h16[lo:hi]
+                block, h = blocks[:hi - lo, :vocab], _operand(hidden[lo:hi])
                 gemm(h, w16, block, hi - lo, vocab, width, b_transposed=True)
                 _ce_rows(block, tgt[lo:hi], row_stats[0, lo:hi], row_stats[1, lo:hi], scale, z_coef, ignore_index)
                 gemm(block, w16, d_hidden[lo:hi], hi - lo, width, vocab)
@@ -192,10 +206,11 @@ class _LinearCrossEntropy(torch.autograd.Function):
 
 def fused_linear_cross_entropy(hidden: Tensor, weight: Tensor, targets: Tensor, normalizer: float,
                                z_loss: float = 0.0, ignore_index: int = -100,
-                               chunk_size: int = 2048) -> tuple[Tensor, Tensor, Tensor]:
+                               chunk_size: int = _CHUNK) -> tuple[Tensor, Tensor, Tensor]:
     """Returns (loss, ce_sum, z_sum): loss = (sum CE + z_loss * sum lse^2) / normalizer
     (fused_ce.py:111-132). hidden (..., H), weight (V, H), targets (...) integer class ids
-    with ignore_index marking unsupervised tokens."""
+    with ignore_index marking unsupervised tokens. A chunk_size is the most tokens whose d logits are in
+    memory at once; without one up to 1.25 GiB of them are, where the device has that."""
     if not hidden.is_cuda:
         raise RuntimeError("fused cross entropy is CUDA-only")
     _same_device(hidden.device, weight=weight, targets=targets)

@@ -206,16 +206,19 @@ def test_rows_with_a_vocabulary_tail(rows, vocab, stride, dtype):
     assert (padded[:, vocab:] == 7).all()
 
 
-@pytest.mark.parametrize("tokens, width, vocab, chunk, keep", [(100, 72, 1003, 33, 1 << 30), (100, 72, 1003, 33, 1), (517, 64, 264, 128, 2 * 264 * 2 * 128)])
+@pytest.mark.parametrize("tokens, width, vocab, chunk, keep", [(100, 72, 1003, 33, 1 << 30), (100, 72, 1003, 33, 1), (517, 64, 264, 128, 2 * 264 * 2 * 128),
+                                                              (100, 72, 1003, None, 1 << 30)])
 @pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32)])
 def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, dtypes):
     """One pass and several, the last one shorter, give the reference's loss and gradients; passes too
-    large for the device's memory are taken back for passes of chunk_size."""
+    large for the device's memory are taken back for passes of the default's tokens (here `chunk`; without one
+    the call names 40)."""
     monkeypatch.setattr(fused_ce, "_KEEP_BYTES", keep)
+    named = {"chunk_size": 40 if chunk is None else fused_ce._Unset(chunk)}
     real, refused, passes = fused_ce.gemm, [], []
 
     def scarce(a, b, c, m, n, k, **kw):
-        if kw.get("a_transposed") and k > chunk and tokens > 500:  # no memory for the larger passes
+        if kw.get("a_transposed") and tokens > 500 and k > chunk:  # no memory for the larger passes
             refused.append(k)
             raise torch.OutOfMemoryError("planted")
         if kw.get("a_transposed"):
@@ -229,10 +232,10 @@ def test_kept_chunks_and_dtypes(monkeypatch, tokens, width, vocab, chunk, keep, 
     targets = torch.randint(0, vocab, (tokens,), generator=g).cuda()
     targets[::7] = -100
     n = float((targets != -100).sum())
-    loss, ce_sum, z_sum = fused_ce.fused_linear_cross_entropy(hidden, weight, targets, n, 1e-3, chunk_size=chunk)
+    loss, ce_sum, z_sum = fused_ce.fused_linear_cross_entropy(hidden, weight, targets, n, 1e-3, **named)
     (3.0 * loss).backward()
     assert refused == ([176] if tokens > 500 else [])
-    assert passes == ([128] * 4 + [5] if tokens > 500 else [100] if keep > 1 else [33, 33, 33, 1])
+    assert passes == ([128] * 4 + [5] if tokens > 500 else [40, 40, 20] if chunk is None else [100] if keep > 1 else [33, 33, 33, 1])
     h, w = (x.detach().double().requires_grad_() for x in (hidden, weight))
     logits = h @ w.t()
     lse = torch.logsumexp(logits, -1)
@@ -305,3 +308,37 @@ def test_gradients_of_a_vocabulary_tail_are_rounded_once(rows, vocab, aligned):
     err[torch.arange(rows), targets] = 0
     _say(f"rows of {vocab}, aligned {aligned}: {err.max().item():.4f} ulp")
     assert err.max() <= 0.5 + 2.0 ** -9
+
+
+def test_chunk_size_bounds_the_memory():
+    """Forward and backward of 8192 tokens in chunks of 256: the d logits in memory are those of 256 tokens,
+    beside the results, the bf16 weight and the fp32 partials of the products."""
+    tokens, width, vocab = 8192, 256, 32000
+    hidden = torch.randn(tokens, width, device="cuda").requires_grad_()
+    weight = (0.05 * torch.randn(vocab, width, device="cuda")).requires_grad_()
+    targets = torch.randint(0, vocab, (tokens,), device="cuda")
+
+    def peak(**kw):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        loss = fused_linear_cross_entropy(hidden, weight, targets, float(tokens), **kw)[0]
+        torch.autograd.grad(loss, (hidden, weight))
+        return torch.cuda.max_memory_allocated() - before
+
+    small, default = peak(chunk_size=256), peak()
+    _say(f"peak {small >> 20} MiB in chunks of 256, {default >> 20} MiB by default")
+    results = 2 * tokens * width * 4 + vocab * width * (2 + 4 + 4)
+    assert small <= results + 256 * vocab * 2 * 2 + (32 << 20)
+    assert default >= tokens * vocab * 2
+
+
+def test_compiled_calls_break_the_graph():
+    """Under torch.compile the call runs as it is, its default and a named chunk_size alike."""
+    hidden = torch.randn(64, 64, dtype=torch.bfloat16, device="cuda").requires_grad_()
+    weight = torch.randn(300, 64, dtype=torch.bfloat16, device="cuda").requires_grad_()
+    targets = torch.randint(0, 300, (64,), device="cuda")
+    for kw in ({}, {"chunk_size": 32}):
+        def step():
+            return fused_linear_cross_entropy(hidden * 2, weight, targets, 64.0, **kw)[0]
+        assert torch.equal(torch.compile(step, backend="eager")(), step())

@@ -2,6 +2,7 @@
 CE row entry point (no GPU)."""
 
 import ctypes
+import inspect
 
 import numpy as np
 import pytest
@@ -134,16 +135,18 @@ def test_cpu_tensors_are_rejected():
         fused_linear_cross_entropy(torch.zeros(4, 8), torch.zeros(16, 8), torch.zeros(4, dtype=torch.long), 1.0)
 
 
-def test_passes_hold_no_more_than_they_may(monkeypatch):
-    """A pass is of at most _KEEP_BYTES of d logits or chunk_size tokens, and passes are as few as that allows."""
+def test_passes_hold_no_more_than_they_may():
+    """A pass is of chunk_size tokens where the caller gives one, whatever fits; else of at most _KEEP_BYTES of
+    d logits or the default's tokens, and passes are as few as that allows."""
     rng = np.random.default_rng(0)
     for _ in range(3000):
         tokens, row_bytes, chunk = (int(2 ** rng.uniform(0, 17)), int(2 ** rng.uniform(8, 24)), int(2 ** rng.uniform(0, 12)))
-        rows = fused_ce._pass_rows(tokens, row_bytes, chunk)
-        most = max(chunk, fused_ce._KEEP_BYTES // row_bytes)
-        assert 1 <= rows <= min(tokens, most), (tokens, row_bytes, chunk, rows)
-        assert -(-tokens // rows) == -(-tokens // most), (tokens, row_bytes, chunk, rows)
-    assert fused_ce._pass_rows(16384, 2 * 65664, 2048) == 8192  # two even passes
-    assert fused_ce._pass_rows(100, 4 << 20, 16) == 100  # (320 fit)
-    monkeypatch.setattr(fused_ce, "_KEEP_BYTES", 1)
-    assert fused_ce._pass_rows(100, 2048, 33) == 33
+        assert fused_ce._pass_rows(tokens, row_bytes, chunk) == min(chunk, tokens)
+        rows = fused_ce._pass_rows(tokens, row_bytes, fused_ce._CHUNK)
+        most = max(2048, fused_ce._KEEP_BYTES // row_bytes)
+        assert 1 <= rows <= min(tokens, most), (tokens, row_bytes, rows)
+        assert -(-tokens // rows) == -(-tokens // most), (tokens, row_bytes, rows)
+    assert fused_ce._pass_rows(16384, 2 * 65664, fused_ce._CHUNK) == 8192  # two even passes
+    assert fused_ce._pass_rows(16384, 2 * 65664, 2048) == 2048
+    default = inspect.signature(fused_ce.fused_linear_cross_entropy).parameters["chunk_size"].default
+    assert default == 2048 and isinstance(default, fused_ce._Unset)

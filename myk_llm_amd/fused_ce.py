@@ -26,6 +26,7 @@ from typing import cast
 
 import torch
 from torch import Tensor
+from torch.autograd import forward_ad
 
 from . import _lib
 from .flash_attn import _DeviceGuard, _dtype_code, _same_device, _stream
@@ -165,12 +166,21 @@ def _loss_of(row_stats: Tensor, scale: float, z_coef: float) -> tuple[Tensor, Te
     return out
 
 
+def _plain(x: Tensor) -> bool:
+    """Whether x's values are the memory behind it: no subclass, mapped or wrapped tensor, no tangent."""
+    return (type(x) is Tensor and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and not torch._C._functorch.is_legacy_batchedtensor(x)
+            and (forward_ad._current_level < 0 or forward_ad.unpack_dual(x).tangent is None))
+
+
 def _scaled(grad: Tensor, upstream: Tensor, dtype: torch.dtype) -> Tensor:
-    """grad * upstream, rounded to grad's type, as dtype."""
-    if (dtype not in _SCALE_DTYPES or upstream.dtype != torch.float32 or upstream.device != grad.device
-            or torch.is_grad_enabled() or torch._C._functorch.is_functorch_wrapped_tensor(upstream)
-            or torch._C._functorch.is_legacy_batchedtensor(upstream)):
-        return grad.mul(upstream).to(dtype)  # a gradient of the gradient, or a mapped one, goes through torch
+    """grad * upstream, rounded to grad's type, as dtype. The kernel takes the gradients as the forward left
+    them; what a hook on saved tensors made of them, a gradient of the gradient, or a mapped or dual one goes
+    through torch."""
+    if (grad.dtype not in (torch.bfloat16, torch.float32) or dtype not in _SCALE_DTYPES or upstream.dtype != torch.float32
+            or upstream.device != grad.device or torch.is_grad_enabled() or not _plain(grad) or not _plain(upstream)
+            or not grad.is_contiguous() or grad.data_ptr() % 16 or upstream.numel() != 1):
+        return grad.mul(upstream).to(dtype)
     out = torch.empty_like(grad, dtype=dtype)
     p = _lib.ScaleParams(grad.data_ptr(), out.data_ptr(), upstream.data_ptr(), grad.numel(), _SCALE_DTYPES[grad.dtype],
                          _SCALE_DTYPES[dtype])

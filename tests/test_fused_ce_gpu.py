@@ -342,3 +342,42 @@ def test_compiled_calls_break_the_graph():
         def step():
             return fused_linear_cross_entropy(hidden * 2, weight, targets, 64.0, **kw)[0]
         assert torch.equal(torch.compile(step, backend="eager")(), step())
+
+
+def _twice_as_far(x):
+    y = x.new_empty(*x.shape[:-1], 2 * x.shape[-1])[..., ::2]
+    return y.copy_(x)
+
+
+@pytest.mark.parametrize("unpack", [lambda x: x.t().contiguous().t(), _twice_as_far, lambda x: _flat_view(x, 1),
+                                    lambda x: x.double(), lambda x: x.cpu().cuda()])
+def test_saved_gradients_may_come_back_in_another_layout(unpack):
+    """A hook on saved tensors may hand the stored gradients back strided, unaligned or in another type."""
+    g = torch.Generator().manual_seed(3)
+    hidden = torch.randn(30, 64, generator=g).to(torch.bfloat16).cuda().requires_grad_()
+    weight = (0.1 * torch.randn(300, 64, generator=g)).cuda().requires_grad_()
+    targets = torch.randint(0, 300, (30,), generator=g).cuda()
+    exp = torch.autograd.grad(3.0 * fused_linear_cross_entropy(hidden, weight, targets, 30.0)[0], (hidden, weight))
+    with torch.autograd.graph.saved_tensors_hooks(lambda x: x, unpack):
+        loss = 3.0 * fused_linear_cross_entropy(hidden, weight, targets, 30.0)[0]
+    got = torch.autograd.grad(loss, (hidden, weight))
+    for a, b in zip(got, exp):
+        assert a.dtype == b.dtype
+        # one rounding of a bf16 product (none of a float64 one)
+        torch.testing.assert_close(a.float(), b.float(), rtol=2.0 ** -8, atol=0)
+
+
+def test_upstream_gradients_of_other_kinds():
+    """A mapped upstream gradient maps the gradients, a dual one gives them its tangent."""
+    hidden = torch.randn(30, 64, device="cuda").to(torch.bfloat16).requires_grad_()
+    weight = (0.1 * torch.randn(300, 64, device="cuda")).requires_grad_()
+    loss = fused_linear_cross_entropy(hidden, weight, torch.randint(0, 300, (30,), device="cuda"), 30.0)[0]
+    (exp,) = torch.autograd.grad(loss, weight, torch.tensor(1.0, device="cuda"), retain_graph=True)
+    factors = torch.tensor([1.0, 2.0, -0.5], device="cuda")
+    (mapped,) = torch.autograd.grad(loss, weight, factors, retain_graph=True, is_grads_batched=True)
+    assert torch.equal(mapped, factors[:, None, None] * exp)
+    with torch.autograd.forward_ad.dual_level():
+        up = torch.autograd.forward_ad.make_dual(torch.tensor(1.0, device="cuda"), torch.tensor(4.0, device="cuda"))
+        (dual,) = torch.autograd.grad(loss, weight, up)
+        primal, tangent = torch.autograd.forward_ad.unpack_dual(dual)
+        assert torch.equal(primal, exp) and tangent is not None and torch.equal(tangent, 4.0 * exp)

@@ -304,7 +304,7 @@ typedef struct mykfa_syrk_params {
  * contiguous last dimension, 16-byte aligned, strides multiples of 8 elements (C fp32: 4). A row is
  * read up to the next multiple of 8 elements: what lies past k must be finite where the other
  * operand has k rows, and zero where both have k columns; the pads of C's rows up to a multiple of
- * 8 columns are stored too (zeros for bf16 without Add).
+ * 8 columns are stored too (bf16: zeros; fp32: what the operands' pads give).
  * symmetric: B = A^T (b ignored, n = m), Add symmetric; only the tiles on and below the diagonal
  * are computed and mirrored, no pad of C is stored, and C and Add need only the alignment of
  * mykfa_syrk.

@@ -134,6 +134,12 @@ __device__ inline void store8(uint16_t* c, s16x8 w, int left, bool vec) {
             if (e < left) c[e] = (uint16_t)w[e];
     }
 }
+// The first `left` of 8 elements, zeros after them.
+__device__ inline s16x8 first8(s16x8 w, int left) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = e < left ? w[e] : (short)0;
+    return w;
+}
 __device__ inline s16x8 load8(const uint16_t* d, int left, bool vec) {
     if (vec && left >= 8) return ld16(d);
     s16x8 w = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -284,8 +290,9 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
             const uint16_t* add = p.add ? p.add + t.bidx * p.d_bs : nullptr;
             uint16_t* cb = static_cast<uint16_t*>(p.c) + t.bidx * p.c_bs;
             pend = full && OUT == OUT_BF16 ? STAGES - 1 : 0;
-            // Columns stored: OUT_BF16 and OUT_ADD fill a row's pad up to a multiple of 8 (B's rows past n are
-            // zero); OUT_SYM stores none.
+            // Columns stored: OUT_BF16 and OUT_ADD fill a row's pad up to a multiple of 8 with zeros, whatever the
+            // operands hold there (an infinity in A's row times the zeros past B's last row is a NaN); OUT_SYM
+            // stores none.
             const int n_end = OUT == OUT_SYM ? p.n : (p.n + 7) & ~7;
 #pragma unroll
             for (int i = 0; i < MI; ++i)
@@ -327,11 +334,15 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
                             wave_fence();
                         }
                         const int r = 8 * q + (lane >> 3), ch = lane & 7, m = mb + r, n = nb + 8 * ch;
-                        const s16x8 y = *reinterpret_cast<const s16x8*>(tr + r % 16 * 64 + ((ch ^ (r & 7)) << 3));
+                        s16x8 y = *reinterpret_cast<const s16x8*>(tr + r % 16 * 64 + ((ch ^ (r & 7)) << 3));
                         if (full || (m < p.m && n < n_end)) {
                             uint16_t* c = cb + (int64_t)m * p.c_rs + n;
-                            if constexpr (OUT == OUT_SYM) store8(c, y, n_end - n, p.c_vec);
-                            else st16(c, y);
+                            if constexpr (OUT == OUT_SYM) {
+                                store8(c, y, n_end - n, p.c_vec);
+                            } else {
+                                if (!full) y = first8(y, p.n - n);
+                                st16(c, y);
+                            }
                         }
                     }
                     if (OUT == OUT_SYM && t.m0 != t.n0) {
@@ -407,15 +418,16 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
     }
 }
 
-// The K splits' fp32 products, summed in order and rounded: 8 columns a lane.
+// The K splits' fp32 products, summed in order and rounded: 8 columns a lane, zeros past n.
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* part, int splits, int64_t stride, uint16_t* c,
-                                                          int64_t c_bs, int64_t c_rs, int batch, int m, int n8,
+                                                          int64_t c_bs, int64_t c_rs, int batch, int m, int n,
                                                           float alpha) {
+    const int n8 = (n + 7) / 8;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t per = (int64_t)m * n8;
     if (idx >= per * batch) return;
-    const int64_t b = idx / per, r = idx % per / n8, n = idx % n8 * 8;
-    const float* s = part + b * splits * stride + (r * n8) * 8 + n;
+    const int64_t b = idx / per, r = idx % per / n8, col = idx % n8 * 8;
+    const float* s = part + b * splits * stride + (r * n8) * 8 + col;
     f32x4 lo = {0.f, 0.f, 0.f, 0.f}, hi = lo;
     for (int i = 0; i < splits; ++i, s += stride) {
         lo += *reinterpret_cast<const f32x4*>(s);
@@ -425,7 +437,7 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const float* part, int
     hi *= alpha;
     const u32x4 w = {BF16::pack2(lo[0], lo[1]), BF16::pack2(lo[2], lo[3]), BF16::pack2(hi[0], hi[1]),
                      BF16::pack2(hi[2], hi[3])};
-    st16(c + b * c_bs + r * c_rs + n, __builtin_bit_cast(s16x8, w));
+    st16(c + b * c_bs + r * c_rs + col, first8(__builtin_bit_cast(s16x8, w), n - (int)col));
 }
 
 template <int WM, int WN, int MI, int NI, int STAGES, int OCC, bool AT, bool BT, int OUT>
@@ -573,7 +585,7 @@ hipError_t launch_gemm(const mykfa_gemm_params& p, void* ws, hipStream_t stream)
         const int64_t lanes = (int64_t)p.batch * p.m * n8;
         hipLaunchKernelGGL(gemm_reduce_kernel, dim3((unsigned)((lanes + 255) / 256)), dim3(256), 0, stream,
                            static_cast<const float*>(ws), plan.splits, (int64_t)p.m * n8 * 8,
-                           static_cast<uint16_t*>(p.c), p.c_batch_stride, p.c_row_stride, p.batch, p.m, n8, p.alpha);
+                           static_cast<uint16_t*>(p.c), p.c_batch_stride, p.c_row_stride, p.batch, p.m, p.n, p.alpha);
         return hipGetLastError();
     }
     if (p.add)

@@ -381,3 +381,16 @@ def test_upstream_gradients_of_other_kinds():
         (dual,) = torch.autograd.grad(loss, weight, up)
         primal, tangent = torch.autograd.forward_ad.unpack_dual(dual)
         assert torch.equal(primal, exp) and tangent is not None and torch.equal(tangent, 4.0 * exp)
+
+
+def test_an_ignored_token_with_infinities_has_no_gradient():
+    """With a vocabulary that 8 does not divide, rows of the d logits have pads, which are read back."""
+    hidden = torch.randn(40, 64, device="cuda").to(torch.bfloat16)
+    hidden[7, 5] = float("inf")
+    hidden.requires_grad_()
+    weight = torch.randn(1003, 64, device="cuda").to(torch.bfloat16).requires_grad_()
+    targets = torch.randint(0, 1003, (40,), device="cuda")
+    targets[7] = -100
+    loss = fused_linear_cross_entropy(hidden, weight, targets, 39.0)[0]
+    (grad,) = torch.autograd.grad(loss, hidden)
+    assert torch.isfinite(loss) and torch.isfinite(grad).all() and (grad[7] == 0).all()

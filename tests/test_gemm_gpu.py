@@ -102,3 +102,20 @@ def test_quarters_past_an_edge(m, n, k):
     x[..., :k] = rows
     gemm(x, w, b, m, n, k)
     _close(b[..., :n], rows.double() @ w[..., :n].double(), k, True)
+
+
+@pytest.mark.parametrize("m, n, k", [(70, 33, 72), (300, 33, 8200), (700, 2500, 4104), (4136, 4099, 136)])
+def test_pads_are_zeros(m, n, k):
+    """Every bf16 result but the symmetric one pads its rows with zeros: with B's pads not a number, with A's
+    rows infinite against the rows that B has not, with an addend whose pads are not a number."""
+    g = torch.Generator().manual_seed(m)
+    a, w, wt = _padded(g, 1, m, k), _padded(g, 1, k, n, fill=float("nan")), _padded(g, 1, n, k)
+    inf = a.clone()
+    inf[0, 1::2, 3] = float("inf")
+    n8 = (n + 7) // 8 * 8
+    assert n8 > n
+    for left, right, kw in ((a, w, {}), (inf, wt, {"b_transposed": True}), (a, w, {"add": _padded(g, 1, m, n, fill=float("nan")), "beta": 1.0})):
+        c = torch.full((1, m, n8), 7.0, dtype=torch.bfloat16, device="cuda")
+        gemm(left, right, c, m, n, k, **kw)
+        assert (c[..., n:] == 0).all()
+        assert not torch.isnan(c[0, 0, :n]).any()

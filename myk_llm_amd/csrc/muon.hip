@@ -13,6 +13,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kMaxParts = 256;  // partial sums of squares per matrix
+constexpr int kMaxBatch = 65535;  // matrices per launch, a grid dimension: more go in several runs
 constexpr int kT = 64;          // transpose tile
 
 int round8(int x) { return (x + 7) & ~7; }
@@ -168,25 +169,20 @@ struct Sizes {
     int M, K;                    // X is (M, K)
     size_t x, g, part;           // bytes of one X buffer, of one G buffer, of the partial sums
 };
-Sizes sizes_of(const mykfa_newton_schulz_params& p) {
+Sizes sizes_of(const mykfa_newton_schulz_params& p) {  // of a run
+    const int batch = p.batch < kMaxBatch ? p.batch : kMaxBatch;
     Sizes s;
     s.M = p.transposed ? p.cols : p.rows;
     s.K = p.transposed ? p.rows : p.cols;
-    s.x = (size_t)p.batch * s.M * row_stride(s.K) * 2;
-    s.g = (size_t)p.batch * s.M * row_stride(s.M) * 2;
-    s.part = (size_t)p.batch * kMaxParts * sizeof(float);
+    s.x = (size_t)batch * s.M * row_stride(s.K) * 2;
+    s.g = (size_t)batch * s.M * row_stride(s.M) * 2;
+    s.part = (size_t)batch * kMaxParts * sizeof(float);
     return s;
 }
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-}  // namespace
-
-size_t newton_schulz_bytes(const mykfa_newton_schulz_params& p) {
-    const Sizes s = sizes_of(p);
-    return 2 * align256(s.x) + 2 * align256(s.g) + align256(s.part);
-}
-
-hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, hipStream_t stream) {
+// Up to kMaxBatch matrices.
+hipError_t run(const mykfa_newton_schulz_params& p, void* ws, hipStream_t stream) {
     const Sizes z = sizes_of(p);
     const int M = z.M, K = z.K, M8 = round8(M), K8 = round8(K), Ms = row_stride(M), Ks = row_stride(K);
     char* w = static_cast<char*>(ws);
@@ -257,6 +253,26 @@ hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, h
     o.obs = n; o.ors = p.cols;
     o.rows = M; o.cols = K; o.owidth = p.transposed ? M : K;
     return copy(o, p.batch, p.transposed, stream);
+}
+
+}  // namespace
+
+size_t newton_schulz_bytes(const mykfa_newton_schulz_params& p) {
+    const Sizes s = sizes_of(p);
+    return 2 * align256(s.x) + 2 * align256(s.g) + align256(s.part);
+}
+
+hipError_t launch_newton_schulz(const mykfa_newton_schulz_params& p, void* ws, hipStream_t stream) {
+    for (int b = 0; b < p.batch; b += kMaxBatch) {
+        mykfa_newton_schulz_params q = p;
+        const int64_t at = (int64_t)b * p.rows * p.cols;
+        q.x = static_cast<const uint16_t*>(p.x) + at;
+        q.out = static_cast<uint16_t*>(p.out) + at;
+        q.batch = p.batch - b < kMaxBatch ? p.batch - b : kMaxBatch;
+        const hipError_t e = run(q, ws, stream);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace mykfa

@@ -119,3 +119,16 @@ def test_pads_are_zeros(m, n, k):
         gemm(left, right, c, m, n, k, **kw)
         assert (c[..., n:] == 0).all()
         assert not torch.isnan(c[0, 0, :n]).any()
+
+
+def test_newton_schulz_of_more_matrices_than_a_grid_dimension():
+    """Matrices of the first run, of the border and of the last one."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn(65537, 8, 16, generator=g, device="cuda", dtype=torch.bfloat16)
+    for steps in (1, 2):
+        out = batched_newton_schulz_orthogonalize(x, steps)
+        assert not torch.isnan(out).any()
+        for b in (0, 32768, 65534, 65535, 65536):
+            exp = om.newton_schulz_reference(x[b].float().cpu(), steps)
+            err = (out[b].float().cpu() - exp).norm() / exp.norm()
+            assert err <= 2.0 ** -9 * 3.45 * steps * 2, (b, err)

@@ -372,8 +372,9 @@ int check_newton_schulz(const mykfa_newton_schulz_params* p) {
         return fail(MYKFA_ERR_INVALID, "negative shape (batch %d, %d x %d) or steps (%d)", p->batch, p->rows, p->cols, p->steps);
     if (!(p->a == p->a) || !(p->b == p->b) || !(p->c == p->c) || !(p->eps == p->eps))
         return fail(MYKFA_ERR_INVALID, "a coefficient or eps is NaN");
-    if (p->rows >= (1 << 23) || p->cols >= (1 << 23))  // 128 rows within a buffer descriptor's 2 GiB
-        return fail(MYKFA_ERR_UNSUPPORTED, "%d x %d: a dimension of 2^23 or more", p->rows, p->cols);
+    // 128 rows, which start 64 elements apart or a multiple of that, within a buffer descriptor's 2 GiB.
+    if (p->rows > (1 << 23) - 64 || p->cols > (1 << 23) - 64)
+        return fail(MYKFA_ERR_UNSUPPORTED, "%d x %d: a dimension above 2^23 - 64", p->rows, p->cols);
     if ((long long)p->batch * p->rows * p->cols == 0) return MYKFA_OK;
     {
         const long long m = p->transposed ? p->cols : p->rows, k = p->transposed ? p->rows : p->cols;

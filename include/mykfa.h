@@ -390,6 +390,10 @@ int mykfa_fwd(const mykfa_fwd_params* p, mykfa_stream_t stream);
  * is then mykfa_fwd (workspace may be NULL). */
 size_t mykfa_fwd_workspace_size(const mykfa_fwd_params* p);
 int mykfa_fwd_ws(const mykfa_fwd_params* p, void* workspace, size_t workspace_bytes, mykfa_stream_t stream);
+/* The same over seqused_k[b] + grown keys: after a mykfa_kv_append of `grown` keys, whose lengths
+ * need no launch of their own (flash_attn.py:486-488). */
+int mykfa_fwd_grown(const mykfa_fwd_params* p, int32_t grown, void* workspace, size_t workspace_bytes,
+                    mykfa_stream_t stream);
 
 /* ---- backward ---------------------------------------------------------------------- */
 /* delta = rowsum(dO * O) in fp32 (the preprocess fused into _bwd_dq_kernel,

@@ -182,6 +182,7 @@ SIGNATURES = {
     "mykfa_fwd": (ctypes.c_int, [ctypes.POINTER(FwdParams), _ptr]),
     "mykfa_fwd_workspace_size": (ctypes.c_size_t, [ctypes.POINTER(FwdParams)]),
     "mykfa_fwd_ws": (ctypes.c_int, [ctypes.POINTER(FwdParams), _ptr, ctypes.c_size_t, _ptr]),
+    "mykfa_fwd_grown": (ctypes.c_int, [ctypes.POINTER(FwdParams), _i32, _ptr, ctypes.c_size_t, _ptr]),
     "mykfa_bwd_preprocess": (ctypes.c_int, [ctypes.POINTER(BwdParams), _ptr]),
     "mykfa_bwd_dkdv": (ctypes.c_int, [ctypes.POINTER(BwdParams), _ptr]),
     "mykfa_bwd_dq": (ctypes.c_int, [ctypes.POINTER(BwdParams), _ptr]),

@@ -425,15 +425,22 @@ size_t mykfa_fwd_workspace_size(const mykfa_fwd_params* p) {
 }
 
 int mykfa_fwd_ws(const mykfa_fwd_params* p, void* workspace, size_t workspace_bytes, mykfa_stream_t stream) {
+    return mykfa_fwd_grown(p, 0, workspace, workspace_bytes, stream);
+}
+
+int mykfa_fwd_grown(const mykfa_fwd_params* p, int32_t grown, void* workspace, size_t workspace_bytes,
+                    mykfa_stream_t stream) {
     int rc = check_fwd(p);
     if (rc) return rc;
+    if (grown < 0 || (grown > 0 && p->seqused_k == nullptr))
+        return fail(MYKFA_ERR_INVALID, "grown (%d) must be >= 0, and needs seqused_k above 0", grown);
     if (p->batch == 0 || p->max_seqlen_q == 0) return ok();
     const int splits = mykfa::fwd_default_splits(*p);
     const size_t need = mykfa::fwd_split_bytes(*p, splits);
     if (need > 0 && (workspace == nullptr || workspace_bytes < need))
         return fail(MYKFA_ERR_WORKSPACE, "mykfa_fwd_ws needs %zu bytes; got %zu", need, workspace_bytes);
     if (need > 0 && !aligned16(workspace)) return fail(MYKFA_ERR_INVALID, "mykfa_fwd_ws: workspace must be 16-byte aligned");
-    return launched(mykfa::launch_fwd(*p, splits, workspace, as_stream(stream)), "mykfa_fwd_ws");
+    return launched(mykfa::launch_fwd(*p, splits, workspace, as_stream(stream), grown), "mykfa_fwd_ws");
 }
 
 int mykfa_bwd_preprocess(const mykfa_bwd_params* p, mykfa_stream_t stream) {

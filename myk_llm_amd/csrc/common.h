@@ -441,7 +441,7 @@ struct SeqInfo {
 
 // flash_attn.py:39-55 (_seq_info).
 __device__ inline SeqInfo seq_info(int b, const int32_t* cu, const int32_t* seqused, int seqlen,
-                                   bool use_seqused) {
+                                   bool use_seqused, int grown = 0) {
     SeqInfo s;
     if (cu != nullptr) {
         int start = cu[b];
@@ -453,7 +453,7 @@ __device__ inline SeqInfo seq_info(int b, const int32_t* cu, const int32_t* sequ
         s.row0 = (int64_t)b * seqlen;
         int len = seqlen;
         if (use_seqused && seqused != nullptr) {  // clamp: never read beyond the cache capacity
-            len = seqused[b];
+            len = seqused[b] + grown;
             len = len < 0 ? 0 : (len > seqlen ? seqlen : len);
         }
         s.len = len;

@@ -42,6 +42,7 @@ struct FwdArgs {
     // Key splits (SPLIT kernels): slots per block, and the fp32 partials of part = sequence *
     // splits + split: unnormalized O [part][head][query][D], then (m, l) [part][head][query].
     int splits;
+    int grown;  // keys of every sequence past seqused_k
     float* ws_o;
     f32x2* ws_ml;
 };
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(NW * 64) void fwd_kernel(FwdArgs a) {
     SeqInfo qs = seq_info(b, a.cu_q, nullptr, a.seqlen_q, false);
     const int tok_base = mblk * tpw * 32;
     if (tok_base >= qs.len) return;
-    SeqInfo ks = seq_info(b, a.cu_k, a.seqused_k, a.seqlen_k, true);
+    SeqInfo ks = seq_info(b, a.cu_k, a.seqused_k, a.seqlen_k, true, a.grown);
     const int q_len = qs.len, k_len = ks.len;
     const int kvh = h_first / a.group;
     const int lo_off = band_lo(k_len, q_len, a.wl);
@@ -350,7 +351,7 @@ __global__ __launch_bounds__(256) void merge_kernel(FwdArgs a, int tpw) {
     const int64_t idx = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;  // (sequence, query, head)
     if (idx >= (int64_t)a.gy * a.seqlen_q * heads) return;
     const int h = (int)(idx % heads), qi = (int)(idx / heads % a.seqlen_q), b = (int)(idx / heads / a.seqlen_q);
-    const SeqInfo ks = seq_info(b, nullptr, a.seqused_k, a.seqlen_k, true);
+    const SeqInfo ks = seq_info(b, nullptr, a.seqused_k, a.seqlen_k, true, a.grown);
     const int n = key_tiles(qi / (tpw * 32) * (tpw * 32), tpw, a.seqlen_q, ks.len, band_lo(ks.len, a.seqlen_q, a.wl),
                             band_hi(ks.len, a.seqlen_q, a.wr), BN).n;
     const int per = split_tiles(n, a.splits);
@@ -468,8 +469,9 @@ int fwd_default_splits(const mykfa_fwd_params& p) {
     return splits < 2 ? 1 : (int)splits;
 }
 
-hipError_t launch_fwd(const mykfa_fwd_params& p, int splits, void* ws, hipStream_t stream) {
+hipError_t launch_fwd(const mykfa_fwd_params& p, int splits, void* ws, hipStream_t stream, int grown) {
     FwdArgs a;
+    a.grown = grown;
     a.splits = splits;
     a.ws_o = static_cast<float*>(ws);
     a.ws_ml = splits > 1 ? reinterpret_cast<f32x2*>(a.ws_o + (size_t)splits * p.batch * p.num_heads * p.max_seqlen_q * p.head_dim)

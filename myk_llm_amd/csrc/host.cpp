@@ -30,7 +30,7 @@ using torch::autograd::variable_list;
 struct Entries {
     decltype(&mykfa_fwd) fwd;
     decltype(&mykfa_fwd_workspace_size) fwd_workspace_size;
-    decltype(&mykfa_fwd_ws) fwd_ws;
+    decltype(&mykfa_fwd_grown) fwd_grown;
     decltype(&mykfa_bwd) bwd;
     decltype(&mykfa_bwd_workspace_per_kv_head) bwd_workspace_per_kv_head;
     decltype(&mykfa_decode) decode;
@@ -98,6 +98,7 @@ struct Seqs {
     int64_t max_q, max_k;
     double scale;
     int64_t wl, wr;
+    int32_t grown = 0;  // keys past seqused
 };
 
 mykfa_fwd_params params(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out, const Tensor& lse,
@@ -165,7 +166,9 @@ std::pair<Tensor, Tensor> forward(const Tensor& q, const Tensor& k, const Tensor
         launch_decode(p, q, nullptr, nullptr);
     } else if (!varlen && q.size(0) * q.size(1) * q.size(2) <= kSplitMaxRows && (bytes = L.fwd_workspace_size(&p)) > 0) {
         const Tensor ws = workspace(bytes, q);
-        check(L.fwd_ws(&p, ws.data_ptr(), bytes, abi(stream_of(q))));
+        check(L.fwd_grown(&p, s.grown, ws.data_ptr(), bytes, abi(stream_of(q))));
+    } else if (s.grown > 0) {
+        check(L.fwd_grown(&p, s.grown, nullptr, 0, abi(stream_of(q))));
     } else {
         check(L.fwd(&p, abi(stream_of(q))));
     }
@@ -352,7 +355,7 @@ PyObject* kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
             const c10::DeviceGuard guard(q.device());
             check(L.kv_append(&p, abi(stream_of(q))));
         }
-        s.seqused = at::add(lens, (int64_t)k.size(1));
+        s.grown = (int32_t)k.size(1);  // (a launch of their addition less: the forward's merge is one more)
         std::tie(out, lse) = forward(q, kc, vc, s);
     }
     if (a[9] != Py_True) return THPVariable_Wrap(out);

@@ -13,7 +13,8 @@ namespace mykfa {
 // alone leave the chip idle.
 int fwd_default_splits(const mykfa_fwd_params& p);
 size_t fwd_split_bytes(const mykfa_fwd_params& p, int splits);
-hipError_t launch_fwd(const mykfa_fwd_params& p, int splits, void* ws, hipStream_t stream);
+// grown: keys of every sequence past seqused_k.
+hipError_t launch_fwd(const mykfa_fwd_params& p, int splits, void* ws, hipStream_t stream, int grown = 0);
 
 hipError_t launch_bwd_preprocess(const mykfa_bwd_params& p, hipStream_t stream);
 hipError_t launch_bwd_dkdv(const mykfa_bwd_params& p, hipStream_t stream);

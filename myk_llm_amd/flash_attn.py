@@ -446,7 +446,7 @@ class _FlashAttn(torch.autograd.Function):
 # --- the native host path (csrc/host.cpp) ---------------------------------------------------
 
 _host = None
-_HOST_ENTRIES = ("fwd", "fwd_workspace_size", "fwd_ws", "bwd", "bwd_workspace_per_kv_head", "decode",
+_HOST_ENTRIES = ("fwd", "fwd_workspace_size", "fwd_grown", "bwd", "bwd_workspace_per_kv_head", "decode",
                  "decode_num_splits", "decode_workspace_size", "kv_append")
 
 

@@ -182,6 +182,15 @@ def test_decode_new_key_rules(L):
     assert b"k_new" in L.mykfa_last_error()
 
 
+def test_grown_lengths_need_the_cached_ones(L):
+    p = good_fwd()
+    assert L.mykfa_fwd_grown(ctypes.byref(p), -1, None, 0, None) == _lib.ERR_INVALID
+    assert L.mykfa_fwd_grown(ctypes.byref(p), 4, None, 0, None) == _lib.ERR_INVALID  # no seqused_k
+    assert b"grown" in L.mykfa_last_error()
+    p.seqused_k, p.batch = 0x60000, 0
+    assert L.mykfa_fwd_grown(ctypes.byref(p), 4, None, 0, None) == _lib.OK  # nothing to do
+
+
 def test_decode_split_heuristic(L):
     # Full 16K caches of a 64-sequence batch: ~1408 keys per split, 12 splits, for one query of
     # a 4-head group and for the 4-query draft alike.

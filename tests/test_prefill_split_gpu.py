@@ -47,3 +47,27 @@ def test_dense_batches_around_the_rule(sq, sk, heads):
     exp, exp_lse = reference_with_lse(q, k, v, True, (-1, -1))
     assert_close(out, exp)
     assert_lse(lse, exp_lse)
+
+
+@pytest.mark.parametrize("nq, heads, kv_heads, d, lens, cap, dtype", [
+    (389, 16, 4, 128, [0], 8192, torch.bfloat16),     # eight slots a block, one or two parts
+    (100, 8, 2, 64, [0, 300, 2, 900], 8192, torch.bfloat16),
+    (40, 4, 4, 32, [8160], 8192, torch.float16),      # keys past the capacity are dropped
+    (500, 2, 1, 256, [17], 4096, torch.bfloat16),
+])
+def test_short_prompts_into_large_caches(nq, heads, kv_heads, d, lens, cap, dtype):
+    print(f"short prompt nq={nq} H={heads}/{kv_heads} D={d} lens={lens} cap={cap}", flush=True)
+    g = torch.Generator().manual_seed(nq)
+    b = len(lens)
+    mk = lambda *s: torch.randn(*s, generator=g).to(dtype)  # noqa: E731
+    q, kc, vc, kn, vn = mk(b, nq, heads, d), mk(b, cap, kv_heads, d), mk(b, cap, kv_heads, d), mk(b, nq, kv_heads, d), mk(b, nq, kv_heads, d)
+    cl = torch.tensor(lens, dtype=torch.int32)
+    exp, exp_lse, exp_k, exp_v = kvcache_reference(q.float(), kc.float(), vc.float(), kn.float(), vn.float(), cl, True, (-1, -1))
+    for index in (torch.int32, torch.int64):  # (int64 lengths: the Python path)
+        kd, vd, seq = kc.cuda(), vc.cuda(), cl.to(index).cuda()
+        out, lse = flash_attn_with_kvcache(q.cuda(), kd, vd, kn.cuda(), vn.cuda(), cache_seqlens=seq, causal=True,
+                                           return_softmax_lse=True)
+        assert_close(out, exp)
+        assert_lse(lse, exp_lse)
+        assert torch.equal(kd.cpu().float(), exp_k.float()) and torch.equal(vd.cpu().float(), exp_v.float())
+        assert torch.equal(seq.cpu(), cl.to(index))

@@ -47,8 +47,12 @@ struct FwdArgs {
     f32x2* ws_ml;
 };
 
-// Tiles a key split holds at least: below it a part costs more in its prologue (Q rows and
-// first tiles landing, ~3 us) and in partials than its tiles take.
+// Tiles per part at least (all but a block's last part), where a sequence is shorter than the capacity that
+// the slots were sized by: more leave slots idle, whose share of an XCD's CUs the others then do not use. GPU
+// time of a prefill of 389 queries of 16 heads of 128 into 8192 rows, behind 500 / 1000 / 1500 / 3000 keys:
+// 26.7 / 30.4 / 31.9 / 34.9 us with 4 (25.7 / 33.9 / 42.2 / 66.1 whole), 30.4 / 31.6 / 33.9 / 34.7 with 6,
+// 32.2 / 33.5 / 34.3 / 36.9 with 8. Numbering all first parts before the second ones loses the L2 that the
+// blocks of one part share (42.6 -> 54.2 us behind 6000 keys).
 constexpr int kMinSplitTiles = 4;
 
 // Key tiles [lo, lo + BN * n) of a workgroup's token blocks: the union over its tpw blocks of
@@ -452,9 +456,11 @@ size_t fwd_split_bytes(const mykfa_fwd_params& p, int splits) {
 // round). Measured (us, at 1 / 128 / 256 / 384 / 448 / 512 / 768 workgroups): 112.7 / 67.0 / 44.8 / 41.5 /
 // 40.2 / 49.1 / 48.3 there (bf16, D 128, 6389 keys), 70.5 / 46.8 / 37.3 / 36.0 / 34.6 / 35.5 / 35.4 with 1000
 // queries of 8 heads on 3000 keys, 44.6 / 44.2 / 32.6 / 30.0 / 29.8 / 30.0 / 32.0 with 2 x 1500 queries of 4
-// heads of 64 on 2000. Parts of fewer than 9 tiles (16 up to D = 64, whose tiles are half the work)
-// cost more in prologues and partials than they save: 2 x 300 queries of 8 heads of 64 on 2000 keys
-// 30.3 whole, 18.3 in four parts, 21.7 in eight; a 512 window 18.4 whole, 21.7 in two.
+// heads of 64 on 2000. These are slots, sized by the most keys that a block can see (the capacity or the
+// window): one for every 9 tiles of them (16 up to D = 64, whose tiles are half the work), since parts shorter
+// than that cost more in prologues and partials than they save: 2 x 300 queries of 8 heads of 64 on 2000 keys
+// 30.3 whole, 18.3 in four slots, 21.7 in eight; a 512 window 18.4 whole, 21.7 in two. A sequence shorter than
+// the capacity spreads its tiles over the slots there are, kMinSplitTiles to a part at least.
 int fwd_default_splits(const mykfa_fwd_params& p) {
     if (p.cu_seqlens_q != nullptr || p.batch <= 0 || p.max_seqlen_q <= 0) return 1;
     const int hpw = gcd_int(p.num_heads / p.num_kv_heads, 4), rows = 4 / hpw * 32, BN = p.head_dim > 128 ? 32 : 64;
@@ -462,7 +468,7 @@ int fwd_default_splits(const mykfa_fwd_params& p) {
     long long span = (long long)p.window_left + p.window_right + rows + BN;  // most keys a block sees
     if (span > p.max_seqlen_k) span = p.max_seqlen_k;
     const long long tiles = (span + BN - 1) / BN;
-    const int least = p.head_dim <= 64 ? 16 : 9;
+    const int least = p.head_dim <= 64 ? 16 : 9;  // of the capacity's tiles per slot
     long long splits = 448 / blocks;
     if (splits > tiles / least) splits = tiles / least;
     if (splits > 64) splits = 64;

@@ -180,8 +180,8 @@ Tensor as_ready(const Tensor& x) { return ready(x) ? x : x.contiguous(); }
 variable_list backward(Tensor dout, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out,
                        const Tensor& lse, const Seqs& s) {
     dout = as_ready(dout);
-    const Tensor dq = at::empty(q.sizes(), q.options()), dk = at::empty(k.sizes(), k.options()),
-                 dv = at::empty(v.sizes(), v.options()), delta = at::empty(lse.sizes(), lse.options());
+    Tensor dq = at::empty(q.sizes(), q.options()), dk = at::empty(k.sizes(), k.options()),
+           dv = at::empty(v.sizes(), v.options()), delta = at::empty(lse.sizes(), lse.options());
     mykfa_bwd_params b{};
     b.fwd = params(q, k, v, out, lse, s);
     b.dout = dout.const_data_ptr();
@@ -194,7 +194,9 @@ variable_list backward(Tensor dout, const Tensor& q, const Tensor& k, const Tens
     strides(dk, b.dk_batch_stride, b.dk_token_stride, b.dk_head_stride);
     strides(dv, b.dv_batch_stride, b.dv_token_stride, b.dv_head_stride);
     if (L.bwd_workspace_per_kv_head(&b) > 0) {
-        // The stored-dS backward plans its passes against the device's memory in Python.
+        // The stored-dS backward plans its passes against the device's memory in Python, with gradients of
+        // its own: these go back first, or they would count against the passes.
+        for (Tensor* x : {&dq, &dk, &dv, &delta}) x->reset();
         PyGILState_STATE g = PyGILState_Ensure();
         const auto wrap = [](const Tensor& x) -> PyObject* { return x.defined() ? THPVariable_Wrap(x) : Py_NewRef(Py_None); };
         PyObject* r = PyObject_CallFunction(py_backward, "NNNNNNNNLLdLL", wrap(dout), wrap(q), wrap(k), wrap(v), wrap(out),

@@ -152,3 +152,26 @@ def test_refusals_and_autograd_from_outside(monkeypatch):
 
     for call in (hooked, twice, unused):
         _same(*_both(monkeypatch, call))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_stored_ds_backward_holds_its_gradients_once(monkeypatch, packed):
+    """Where the backward is planned in Python the native one keeps nothing beside it: the same peak."""
+    g = torch.Generator().manual_seed(0)
+    n = 2048
+    q, k, v = (x.requires_grad_() for x in _qkv(g, (n,) if packed else (1, n), 16, 4, 128, torch.bfloat16, "plain"))
+    dout = torch.randn(q.shape, generator=g).to(torch.bfloat16).cuda()
+    cu = torch.tensor([0, 500, n], dtype=torch.int32, device="cuda")
+
+    def call():
+        out = flash_attn_varlen_func(q, k, v, cu, cu, n, n, causal=True) if packed else flash_attn_func(q, k, v, causal=True)
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        grads = torch.autograd.grad(out, (q, k, v), dout)
+        torch.cuda.synchronize()
+        return torch.cuda.max_memory_allocated() - before, grads
+
+    (got, a), (exp, b) = _both(monkeypatch, call)
+    _same(a, b)
+    assert got <= exp, (got, exp)

@@ -56,6 +56,15 @@ void check(int status) {
     throw e;
 }
 
+// Other Python threads run while this one allocates and launches, which can wait for the device. (The
+// arguments are the caller's, who holds them until the call returns.)
+struct WithoutGil {
+    PyThreadState* state = PyEval_SaveThread();
+    WithoutGil() = default;
+    WithoutGil(const WithoutGil&) = delete;
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
 bool plain(const Tensor& x) {
     return x.is_cuda() && x.layout() == at::kStrided && !at::isTensorSubclassLike(x) && !x._fw_grad(0).defined();
 }
@@ -173,6 +182,37 @@ std::pair<Tensor, Tensor> forward(const Tensor& q, const Tensor& k, const Tensor
         check(L.fwd(&p, abi(stream_of(q))));
     }
     return {out, lse};
+}
+
+// (O, LSE) of flash_attn_with_kvcache: k and v appended to the caches, q over the grown lengths.
+std::pair<Tensor, Tensor> cached(const Tensor& q, const Tensor& kc, const Tensor& vc, const Tensor& k, const Tensor& v, Seqs& s) {
+    const c10::DeviceGuard guard(q.device());
+    const int64_t b = q.size(0), nq = q.size(1);
+    if (nq <= kDecodeMaxQ) {
+        const Tensor out = at::empty(q.sizes(), q.options());
+        const Tensor lse = at::empty({q.size(2), b * nq}, q.options().dtype(at::kFloat));
+        launch_decode(params(q, kc, vc, out, lse, s), q, &k, &v);
+        return {out, lse};
+    }
+    mykfa_kv_append_params p{};
+    p.k_cache = kc.data_ptr();
+    p.v_cache = vc.data_ptr();
+    p.k_new = k.const_data_ptr();
+    p.v_new = v.const_data_ptr();
+    p.cache_seqlens = static_cast<const int32_t*>(s.seqused.const_data_ptr());
+    strides(kc, p.kc_batch_stride, p.kc_token_stride, p.kc_head_stride);
+    strides(vc, p.vc_batch_stride, p.vc_token_stride, p.vc_head_stride);
+    strides(k, p.kn_batch_stride, p.kn_token_stride, p.kn_head_stride);
+    strides(v, p.vn_batch_stride, p.vn_token_stride, p.vn_head_stride);
+    p.batch = (int32_t)b;
+    p.seqlen_new = (int32_t)k.size(1);
+    p.capacity = (int32_t)kc.size(1);
+    p.num_kv_heads = (int32_t)k.size(2);
+    p.head_dim = (int32_t)k.size(3);
+    p.dtype = k.scalar_type() == at::kBFloat16 ? MYKFA_BF16 : MYKFA_FP16;
+    check(L.kv_append(&p, abi(stream_of(q))));
+    s.grown = (int32_t)k.size(1);  // (a launch of their addition less: the forward's merge is one more)
+    return forward(q, kc, vc, s);
 }
 
 Tensor as_ready(const Tensor& x) { return ready(x) ? x : x.contiguous(); }
@@ -297,11 +337,14 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!PyBool_Check(a[10])) Py_RETURN_NOTIMPLEMENTED;
     const bool with_lse = a[10] == Py_True;
     variable_list r;
-    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) {
-        r = FlashAttn::apply(q, k, v, &s, with_lse);
-    } else {
-        auto [out, lse] = forward(q, k, v, s);
-        r = {out, lse};
+    {
+        const WithoutGil threads;
+        if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) {
+            r = FlashAttn::apply(q, k, v, &s, with_lse);
+        } else {
+            auto [out, lse] = forward(q, k, v, s);
+            r = {out, lse};
+        }
     }
     if (!with_lse) return THPVariable_Wrap(r[0]);
     return Py_BuildValue("NN", THPVariable_Wrap(r[0]), THPVariable_Wrap(r[1]));
@@ -329,36 +372,11 @@ PyObject* kvcache(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!window_arg(a[7], a[6] == Py_True, s.wl, s.wr) || !PyBool_Check(a[6]) || !PyBool_Check(a[9]) ||
         !scale_arg(a[8], q.size(-1), s.scale))
         Py_RETURN_NOTIMPLEMENTED;
-    const at::NoGradGuard no_grad;
     Tensor out, lse;
-    if (nq <= kDecodeMaxQ) {
-        out = at::empty(q.sizes(), q.options());
-        lse = at::empty({q.size(2), b * nq}, q.options().dtype(at::kFloat));
-        const c10::DeviceGuard guard(q.device());
-        launch_decode(params(q, kc, vc, out, lse, s), q, &k, &v);
-    } else {
-        mykfa_kv_append_params p{};
-        p.k_cache = kc.data_ptr();
-        p.v_cache = vc.data_ptr();
-        p.k_new = k.const_data_ptr();
-        p.v_new = v.const_data_ptr();
-        p.cache_seqlens = static_cast<const int32_t*>(lens.const_data_ptr());
-        strides(kc, p.kc_batch_stride, p.kc_token_stride, p.kc_head_stride);
-        strides(vc, p.vc_batch_stride, p.vc_token_stride, p.vc_head_stride);
-        strides(k, p.kn_batch_stride, p.kn_token_stride, p.kn_head_stride);
-        strides(v, p.vn_batch_stride, p.vn_token_stride, p.vn_head_stride);
-        p.batch = (int32_t)b;
-        p.seqlen_new = (int32_t)k.size(1);
-        p.capacity = (int32_t)cap;
-        p.num_kv_heads = (int32_t)k.size(2);
-        p.head_dim = (int32_t)k.size(3);
-        p.dtype = k.scalar_type() == at::kBFloat16 ? MYKFA_BF16 : MYKFA_FP16;
-        {
-            const c10::DeviceGuard guard(q.device());
-            check(L.kv_append(&p, abi(stream_of(q))));
-        }
-        s.grown = (int32_t)k.size(1);  // (a launch of their addition less: the forward's merge is one more)
-        std::tie(out, lse) = forward(q, kc, vc, s);
+    {
+        const WithoutGil threads;
+        const at::NoGradGuard no_grad;
+        std::tie(out, lse) = cached(q, kc, vc, k, v, s);
     }
     if (a[9] != Py_True) return THPVariable_Wrap(out);
     return Py_BuildValue("NN", THPVariable_Wrap(out), THPVariable_Wrap(lse));

@@ -2,6 +2,8 @@
 it accepts, and the same answer from autograd where it is looked at from outside (hooks on saved
 tensors, a second backward, gradients of gradients, mapped and forward-mode gradients)."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -175,3 +177,57 @@ def test_stored_ds_backward_holds_its_gradients_once(monkeypatch, packed):
     (got, a), (exp, b) = _both(monkeypatch, call)
     _same(a, b)
     assert got <= exp, (got, exp)
+
+
+def test_launches_run_without_the_interpreter_lock(monkeypatch):
+    """The entry that the native path asks for the number of decode splits is replaced by the interpreter's own
+    question whether this thread holds its lock; what it answers arrives at the next entry."""
+    g = torch.Generator().manual_seed(0)
+    q, k, v = _qkv(g, (2, 3), 4, 2, 64, torch.bfloat16, "plain")
+    caches = torch.zeros(2, 2, 64, 2, 64, dtype=torch.bfloat16, device="cuda")
+    lens = torch.zeros(2, dtype=torch.int32, device="cuda")
+    held = []
+
+    def size(*args):
+        held.append(args[-1])
+        return 16
+
+    entries = {"decode_num_splits": ctypes.pythonapi.PyGILState_Check,
+               "decode_workspace_size": ctypes.CFUNCTYPE(ctypes.c_size_t, *[ctypes.c_int32] * 5)(size),
+               "decode": ctypes.CFUNCTYPE(ctypes.c_int, *[ctypes.c_void_p] * 2, ctypes.c_size_t, ctypes.c_void_p)(lambda *a: 0)}
+    lib = fa._lib.lib()
+    monkeypatch.setattr(fa, "_host", None)
+    mod = fa._native()
+    try:
+        mod.setup(*(ctypes.cast(entries.get(n) or getattr(lib, f"mykfa_{n}"), ctypes.c_void_p).value for n in fa._HOST_ENTRIES),
+                  fa._lib.check, fa._backward_launch)
+        flash_attn_with_kvcache(q, *caches, k, v, cache_seqlens=lens)
+        flash_attn_func(q, k, v)
+        flash_attn_func(q.requires_grad_(), k, v)
+    finally:
+        fa._host = None
+        fa._native()
+    assert held == [0, 0, 0]
+
+
+def test_errors_of_the_library_and_of_hooks_reach_the_caller(monkeypatch):
+    g = torch.Generator().manual_seed(0)
+    q, k, v = (x.requires_grad_() for x in _qkv(g, (1, 40), 4, 2, 64, torch.bfloat16, "plain"))
+
+    def not_a_scale():
+        flash_attn_func(q, k, v, softmax_scale=float("nan"))
+
+    def not_a_scale_without_gradients():
+        with torch.no_grad():
+            not_a_scale()
+
+    def hook():
+        def pack(x):
+            raise LookupError("no room")
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda x: x):
+            flash_attn_func(q, k, v)
+
+    for call, kind in ((not_a_scale, fa._lib.MykfaError), (not_a_scale_without_gradients, fa._lib.MykfaError), (hook, LookupError)):
+        got, exp = _both(monkeypatch, lambda call=call: _error(call))
+        assert got is exp is kind
+    assert torch.isfinite(flash_attn_func(q, k, v)).all()

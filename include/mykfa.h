@@ -391,7 +391,7 @@ int mykfa_fwd(const mykfa_fwd_params* p, mykfa_stream_t stream);
 size_t mykfa_fwd_workspace_size(const mykfa_fwd_params* p);
 int mykfa_fwd_ws(const mykfa_fwd_params* p, void* workspace, size_t workspace_bytes, mykfa_stream_t stream);
 /* The same over seqused_k[b] + grown keys: after a mykfa_kv_append of `grown` keys, whose lengths
- * need no launch of their own (flash_attn.py:486-488). */
+ * need no launch of their own (flash_attn.py:486-488). Without a workspace no keys are split. */
 int mykfa_fwd_grown(const mykfa_fwd_params* p, int32_t grown, void* workspace, size_t workspace_bytes,
                     mykfa_stream_t stream);
 

@@ -425,6 +425,8 @@ size_t mykfa_fwd_workspace_size(const mykfa_fwd_params* p) {
 }
 
 int mykfa_fwd_ws(const mykfa_fwd_params* p, void* workspace, size_t workspace_bytes, mykfa_stream_t stream) {
+    if (workspace == nullptr && mykfa_fwd_workspace_size(p) > 0)
+        return fail(MYKFA_ERR_WORKSPACE, "mykfa_fwd_ws needs %zu bytes; got none", mykfa_fwd_workspace_size(p));
     return mykfa_fwd_grown(p, 0, workspace, workspace_bytes, stream);
 }
 
@@ -435,9 +437,9 @@ int mykfa_fwd_grown(const mykfa_fwd_params* p, int32_t grown, void* workspace, s
     if (grown < 0 || (grown > 0 && p->seqused_k == nullptr))
         return fail(MYKFA_ERR_INVALID, "grown (%d) must be >= 0, and needs seqused_k above 0", grown);
     if (p->batch == 0 || p->max_seqlen_q == 0) return ok();
-    const int splits = mykfa::fwd_default_splits(*p);
+    const int splits = workspace == nullptr ? 1 : mykfa::fwd_default_splits(*p);
     const size_t need = mykfa::fwd_split_bytes(*p, splits);
-    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
+    if (need > 0 && workspace_bytes < need)
         return fail(MYKFA_ERR_WORKSPACE, "mykfa_fwd_ws needs %zu bytes; got %zu", need, workspace_bytes);
     if (need > 0 && !aligned16(workspace)) return fail(MYKFA_ERR_INVALID, "mykfa_fwd_ws: workspace must be 16-byte aligned");
     return launched(mykfa::launch_fwd(*p, splits, workspace, as_stream(stream), grown), "mykfa_fwd_ws");

@@ -174,8 +174,13 @@ std::pair<Tensor, Tensor> forward(const Tensor& q, const Tensor& k, const Tensor
     if (!varlen && s.max_q > 0 && s.max_q <= kDecodeMaxQ) {
         launch_decode(p, q, nullptr, nullptr);
     } else if (!varlen && q.size(0) * q.size(1) * q.size(2) <= kSplitMaxRows && (bytes = L.fwd_workspace_size(&p)) > 0) {
-        const Tensor ws = workspace(bytes, q);
-        check(L.fwd_grown(&p, s.grown, ws.data_ptr(), bytes, abi(stream_of(q))));
+        Tensor ws;
+        try {
+            ws = workspace(bytes, q);
+        } catch (const c10::OutOfMemoryError&) {
+            bytes = 0;  // the keys then stay whole
+        }
+        check(L.fwd_grown(&p, s.grown, bytes ? ws.data_ptr() : nullptr, bytes, abi(stream_of(q))));
     } else if (s.grown > 0) {
         check(L.fwd_grown(&p, s.grown, nullptr, 0, abi(stream_of(q))));
     } else {

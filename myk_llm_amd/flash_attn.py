@@ -243,8 +243,11 @@ def _forward(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Optional[Tensor], cu
         elif (not varlen and shape[0] * shape[1] * shape[2] <= _SPLIT_MAX_ROWS
               and (nbytes := L.mykfa_fwd_workspace_size(ctypes.byref(p)))):
             # Too few query blocks to fill the chip: their keys are split, partials merged.
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            _lib.check(L.mykfa_fwd_ws(ctypes.byref(p), ws.data_ptr(), nbytes, _stream(dev)))
+            try:
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            except torch.OutOfMemoryError:
+                ws, nbytes = None, 0  # the keys then stay whole
+            _lib.check(L.mykfa_fwd_grown(ctypes.byref(p), 0, _ptr(ws), nbytes, _stream(dev)))
         else:
             _lib.check(L.mykfa_fwd(ctypes.byref(p), _stream(dev)))
     return out, lse

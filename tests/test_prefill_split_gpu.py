@@ -71,3 +71,27 @@ def test_short_prompts_into_large_caches(nq, heads, kv_heads, d, lens, cap, dtyp
         assert_lse(lse, exp_lse)
         assert torch.equal(kd.cpu().float(), exp_k.float()) and torch.equal(vd.cpu().float(), exp_v.float())
         assert torch.equal(seq.cpu(), cl.to(index))
+
+
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])  # the native path, the Python one
+def test_no_memory_for_the_parts(index):
+    """Where the device has no room for the partials the keys stay whole."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    mk = lambda *s: torch.randn(*s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    q, kc, vc, kn, vn = mk(1, 389, 16, 128), mk(1, 8192, 4, 128), mk(1, 8192, 4, 128), mk(1, 389, 4, 128), mk(1, 389, 4, 128)
+    lens = torch.tensor([6000], dtype=index, device="cuda")
+    call = lambda: flash_attn_with_kvcache(q, kc, vc, kn, vn, cache_seqlens=lens, causal=True)  # noqa: E731
+    exp = call()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    before = torch.cuda.memory_stats()["num_ooms"]
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / total)
+    try:
+        got = call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.cuda.memory_stats()["num_ooms"] > before  # 26 MB of partials did not fit
+    assert_close(got, exp)
+    del got
+    assert torch.equal(call(), exp)

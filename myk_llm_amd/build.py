@@ -15,6 +15,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import warnings
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -62,13 +63,22 @@ def _compile(hipcc: str, src: Path) -> Path:
     return obj
 
 
-def _build_host() -> None:
+def _build_host() -> bool:
+    """False, with a warning, where there is no host compiler or torch came without its headers: the kernels
+    need neither, and without _host.so the attention calls take their Python path."""
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
 
+    cxx = os.environ.get("CXX", "g++")
+    headers = (f"{sysconfig.get_paths()['include']}/Python.h", f"{include_paths()[0]}/torch/csrc/autograd/custom_function.h")
+    missing = [h for h in headers if not os.path.exists(h)] + ([] if shutil.which(cxx) else [cxx])
+    if missing:
+        HOST.unlink(missing_ok=True)
+        warnings.warn(f"{HOST.name} is not built: {', '.join(missing)} not found", RuntimeWarning, stacklevel=2)
+        return False
     tmp = HOST.with_suffix(".so.tmp")
     rocm = Path(_hipcc()).resolve().parent.parent
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f"-I{p}" for p in include_paths()), f"-I{sysconfig.get_paths()['include']}", f"-I{rocm / 'include'}",
@@ -78,6 +88,7 @@ def _build_host() -> None:
     if res.returncode != 0:
         raise RuntimeError(f"{cmd[0]} failed on host.cpp:\n{res.stderr}")
     os.replace(tmp, HOST)
+    return True
 
 
 def build(verbose: bool = True) -> Path:
@@ -90,7 +101,7 @@ def build(verbose: bool = True) -> Path:
     with concurrent.futures.ThreadPoolExecutor(workers + 1) as pool:
         host = pool.submit(_build_host)
         objs = list(pool.map(lambda s: _compile(hipcc, s), sources))
-        host.result()
+        native = host.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -98,7 +109,7 @@ def build(verbose: bool = True) -> Path:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB)
     if verbose:
-        print(f"built {LIB} from {len(sources)} sources for {ARCH}, and {HOST}")
+        print(f"built {LIB} from {len(sources)} sources for {ARCH}" + (f", and {HOST}" if native else ""))
     return LIB
 
 

@@ -33,6 +33,7 @@ from __future__ import annotations
 import ctypes
 import math
 import os
+import warnings
 from typing import Optional
 
 import torch
@@ -453,17 +454,30 @@ _HOST_ENTRIES = ("fwd", "fwd_workspace_size", "fwd_grown", "bwd", "bwd_workspace
                  "decode_num_splits", "decode_workspace_size", "kv_append")
 
 
+class _NoHost:
+    """Stands in for an extension that was not built here: every call takes the Python path."""
+
+    @staticmethod
+    def attention(*args):
+        return NotImplemented
+
+    kvcache = attention
+
+
 def _native():
     """The extension that makes the plain calls (GPU tensors as the kernels read them): it answers
-    NotImplemented to every other, which then takes the code below."""
+    NotImplemented to every other, which then takes the code below. Where it is missing or made for another
+    torch, all of them do: the same kernels, with more host time per call."""
     global _host
     if _host is None:
         L = _lib.lib()
         try:
             from . import _host as mod
         except ImportError as e:
-            raise RuntimeError("myk_llm_amd/_host.so is missing or does not load: build it first "
-                               "(python -m myk_llm_amd.build)") from e
+            warnings.warn(f"myk_llm_amd/_host.so is missing or does not load ({e}): attention calls take more host "
+                          "time; build it with python -m myk_llm_amd.build", RuntimeWarning, stacklevel=3)
+            _host = _NoHost
+            return _host
         mod.setup(*(ctypes.cast(getattr(L, f"mykfa_{n}"), ctypes.c_void_p).value for n in _HOST_ENTRIES),
                   _lib.check, _backward_launch)
         _host = mod

@@ -4,11 +4,15 @@ each documented status code (flash_attn.py:336-346, :476-477) without touching a
 
 import ctypes
 import re
+import sys
 from pathlib import Path
 
 import pytest
+import torch.utils.cpp_extension
 
-from myk_llm_amd import _lib
+import myk_llm_amd
+from myk_llm_amd import _lib, build
+from myk_llm_amd import flash_attn as fa
 
 HEADER = Path(__file__).resolve().parents[1] / "include" / "mykfa.h"
 
@@ -222,6 +226,30 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setenv("MYKFA_LIB", str(tmp_path / "nope.so"))
     with pytest.raises(RuntimeError, match="no fallback"):
         _lib.lib()
+
+
+def test_missing_host_extension_takes_the_python_path(monkeypatch, L):
+    monkeypatch.setattr(fa, "_host", None)
+    monkeypatch.delattr(myk_llm_amd, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "myk_llm_amd._host", None)  # importing it raises ImportError
+    with pytest.warns(RuntimeWarning, match="_host.so"):
+        mod = fa._native()
+    assert mod.attention() is NotImplemented and mod.kvcache(1, 2) is NotImplemented
+    assert fa._native() is mod  # one warning
+
+
+@pytest.mark.parametrize("missing", ["compiler", "headers"])
+def test_kernels_build_without_the_host_extension(monkeypatch, tmp_path, missing):
+    stale = tmp_path / "_host.so"
+    stale.write_bytes(b"made for another torch")
+    monkeypatch.setattr(build, "HOST", stale)
+    if missing == "compiler":
+        monkeypatch.setenv("CXX", str(tmp_path / "no-such-compiler"))
+    else:
+        monkeypatch.setattr(torch.utils.cpp_extension, "include_paths", lambda *a, **k: [str(tmp_path)])
+    with pytest.warns(RuntimeWarning, match="not built"):
+        assert build._build_host() is False
+    assert not stale.exists()
 
 
 def _bwd_params(head_dim, window_left=_lib.UNBOUNDED, window_right=0):

@@ -13,18 +13,33 @@ from myk_llm_amd import flash_attn_func, flash_attn_varlen_func, flash_attn_with
 pytestmark = pytest.mark.gpu
 
 
-class _Never:
-    @staticmethod
-    def attention(*a):
-        return NotImplemented
+class _Recorded:
+    """The extension, noting for each call whether it took it."""
 
-    kvcache = attention
+    def __init__(self):
+        self.mod, self.took = fa._native(), []
+
+    def _note(self, r):
+        self.took.append(r is not NotImplemented)
+        return r
+
+    def attention(self, *a):
+        return self._note(self.mod.attention(*a))
+
+    def kvcache(self, *a):
+        return self._note(self.mod.kvcache(*a))
 
 
-def _both(monkeypatch, call):
-    got = call()
+def _both(monkeypatch, call, native=None):
+    """The call's results as it is, and with the Python path alone. native: whether the first is one that the
+    extension takes."""
     with monkeypatch.context() as m:
-        m.setattr(fa, "_host", _Never)
+        recorded = _Recorded()
+        m.setattr(fa, "_host", recorded)
+        got = call()
+        assert native is None or (recorded.took and all(t == native for t in recorded.took)), recorded.took
+    with monkeypatch.context() as m:
+        m.setattr(fa, "_host", fa._NoHost)
         return got, call()
 
 
@@ -70,7 +85,7 @@ def test_attention_bits(monkeypatch, form, packed, d, dtype, needs, with_lse):
         ins = [x for x in (q, k, v) if x.requires_grad]
         return (*(r if with_lse else (r,)), *(torch.autograd.grad(out, ins, dout) if ins else ()))
 
-    _same(*_both(monkeypatch, call))
+    _same(*_both(monkeypatch, call, native=form != "unaligned"))
 
 
 @pytest.mark.parametrize("nq, lens, with_lse", [(1, [0, 200], False), (16, [3, 77], True), (17, [0, 200], True), (40, [250, 1], False)])
@@ -86,7 +101,7 @@ def test_kvcache_bits(monkeypatch, nq, lens, with_lse, index):
         r = flash_attn_with_kvcache(q, kc, vc, k, v, cache_seqlens=cl, causal=True, return_softmax_lse=with_lse)
         return (*(r if with_lse else (r,)), kc, vc)
 
-    _same(*_both(monkeypatch, call))
+    _same(*_both(monkeypatch, call, native=index == torch.int32))
 
 
 def _error(call):
@@ -153,7 +168,7 @@ def test_refusals_and_autograd_from_outside(monkeypatch):
                 torch.tensor(lse.requires_grad))
 
     for call in (hooked, twice, unused):
-        _same(*_both(monkeypatch, call))
+        _same(*_both(monkeypatch, call, native=True))
 
 
 @pytest.mark.parametrize("packed", [False, True])
@@ -174,7 +189,7 @@ def test_stored_ds_backward_holds_its_gradients_once(monkeypatch, packed):
         torch.cuda.synchronize()
         return torch.cuda.max_memory_allocated() - before, grads
 
-    (got, a), (exp, b) = _both(monkeypatch, call)
+    (got, a), (exp, b) = _both(monkeypatch, call, native=True)
     _same(a, b)
     assert got <= exp, (got, exp)
 

@@ -82,13 +82,22 @@ struct Operand {
         part = gemm_part<TR>(mn, k, r0, R);
         base = reinterpret_cast<uint64_t>(p + (int64_t)part.row0 * rs + part.col0);
     }
-    // This wave's loads of K stage kt into the tile at LDS address lds. Rows past the matrix read
-    // zero through the descriptor; chunks past K through their offset.
-    __device__ inline void issue(int kt, uint32_t lds, int wave, int lane) const {
+    struct Stage {
+        i32x4 rsrc;
+        int left;  // columns of K from it on
+    };
+    Stage next;
+    __device__ inline Stage stage(int kt) const {
         const GemmSpan s = gemm_span<TR>(part, (int)rs, kt);
-        const i32x4 rsrc = buffer_rsrc32(base + ((uint64_t)(unsigned)s.row * (uint64_t)rs + (unsigned)s.col) * 2, s.bytes);
+        return Stage{buffer_rsrc32(base + ((uint64_t)(unsigned)s.row * (uint64_t)rs + (unsigned)s.col) * 2, s.bytes),
+                     part.cols - s.col};
+    }
+    // This wave's loads of a stage into the tile at LDS address lds. Rows past the matrix read
+    // zero through the descriptor; chunks past K through their offset.
+    __device__ inline void issue(const Stage& s, uint32_t lds, int wave, int lane) const {
+        const i32x4 rsrc = s.rsrc;
         if constexpr (!TR) {
-            const int left = part.cols - s.col;
+            const int left = s.left;
             if (left < kBK) {
 #pragma unroll
                 for (int j = 0; j < LOADS; ++j) {
@@ -176,6 +185,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
             int r = (int)((sqrtf(8.0f * (float)x + 1.0f) - 1.0f) * 0.5f);
             while (r * (r + 1) / 2 > x) --r;
             while ((r + 1) * (r + 2) / 2 <= x) ++r;
+            r = __builtin_amdgcn_readfirstlane(r);
             return GemmTile{bidx, bidx, r * BM, (x - r * (r + 1) / 2) * BN, 0, p.g.stages};
         } else {
             return gemm_tile(p.g, p.k, unit, BM, BN);
@@ -196,11 +206,20 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
     };
     enter();
     const uint32_t lds0 = lds_addr(&smem[0]);
+    // The symmetric products and the smallest tiles compute the next stage's descriptors before they wait for
+    // the one before: with a CU to themselves, the time from a stage's landing to the next one's loads is their
+    // chain (symmetric 9 x 1024 x 4096 60.3 -> 59.0 us, 9 x 512 x 2048 21.1 -> 19.6, 1 x 1024 x 4096 34.6 -> 32.5).
+    // The 256 x 256 tiles lose by it (8192 x 1024 x 65536 922 -> 942: more scalar registers spilled).
+    constexpr bool kAhead = OUT == OUT_SYM || NW == 2;
+    auto prepare = [&]() {
+        oa.next = oa.stage(lt.kt0 + lk);
+        ob.next = ob.stage(lt.kt0 + lk);
+    };
     auto issue = [&]() {
         if (lu >= end) return;
         const uint32_t at = lds0 + (uint32_t)(lslot * SLOT * 2);
-        oa.issue(lt.kt0 + lk, at, wave, lane);
-        ob.issue(lt.kt0 + lk, at + BM * kBK * 2, wave, lane);
+        oa.issue(kAhead ? oa.next : oa.stage(lt.kt0 + lk), at, wave, lane);
+        ob.issue(kAhead ? ob.next : ob.stage(lt.kt0 + lk), at + BM * kBK * 2, wave, lane);
         ++ahead;
         lslot = lslot + 1 == STAGES ? 0 : lslot + 1;
         if (++lk == lt.nk) {
@@ -213,7 +232,10 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
         }
     };
 #pragma unroll
-    for (int s = 0; s < STAGES; ++s) issue();
+    for (int s = 0; s < STAGES; ++s) {
+        if (kAhead) prepare();
+        issue();
+    }
 
     f32x16 acc[MI][NI];
     s16x8 av[2][MI], bv[2][NI];
@@ -270,6 +292,7 @@ __global__ __launch_bounds__(WM * WN * 64, OCC) void gemm_kernel(GemmArgs p) {
             slot = slot + 1 == STAGES ? 0 : slot + 1;
             const bool more = ahead > 0;
             if (more) {
+                if (kAhead) prepare();
                 landed();
                 if (NW < 8 || wave < NW / 2) issue();
                 read(0, 0);

@@ -22,6 +22,7 @@ tokens as _KEEP_BYTES of d logits do (the default's 2048 where the device's memo
 from __future__ import annotations
 
 import ctypes
+import operator
 from typing import cast
 
 import torch
@@ -75,7 +76,7 @@ def _pass_rows(tokens: int, row_bytes: int, chunk_size: int) -> int:
     even passes over all of them, whole 256-row tiles where that fits, of at most _KEEP_BYTES of d logits or
     the default's tokens, whichever is more."""
     if not isinstance(chunk_size, _Unset):
-        return int(min(chunk_size, tokens))
+        return min(operator.index(chunk_size), tokens)
     most = max(chunk_size, _KEEP_BYTES // row_bytes)
     passes = -(-tokens // most)
     return min(tokens, most, (-(-tokens // passes) + 255) // 256 * 256)

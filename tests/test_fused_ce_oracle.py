@@ -149,5 +149,7 @@ def test_passes_hold_no_more_than_they_may():
     assert fused_ce._pass_rows(16384, 2 * 65664, fused_ce._CHUNK) == 8192  # two even passes
     assert fused_ce._pass_rows(16384, 2 * 65664, 2048) == 2048
     assert type(fused_ce._pass_rows(7, 64, True)) is int and fused_ce._pass_rows(7, 64, np.int64(3)) == 3
+    with pytest.raises(TypeError):
+        fused_ce._pass_rows(7, 64, 7.0)
     default = inspect.signature(fused_ce.fused_linear_cross_entropy).parameters["chunk_size"].default
     assert default == 2048 and isinstance(default, fused_ce._Unset)

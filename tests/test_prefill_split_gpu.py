@@ -85,13 +85,20 @@ def test_no_memory_for_the_parts(index):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
-    before = torch.cuda.memory_stats()["num_ooms"]
-    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / total)
+    filler = []
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (24 << 20)) / total)
     try:
+        room = torch.empty(4 << 20, dtype=torch.uint8, device="cuda")  # for O and the LSE
+        try:
+            while True:  # no 10 MB in one piece are left, and so no 26, the partials, with the room's 4
+                filler.append(torch.empty(10 << 20, dtype=torch.uint8, device="cuda"))
+        except torch.OutOfMemoryError:
+            del room
+        before = torch.cuda.memory_stats()["num_ooms"]
         got = call()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
-    assert torch.cuda.memory_stats()["num_ooms"] > before  # 26 MB of partials did not fit
+    assert torch.cuda.memory_stats()["num_ooms"] > before
     assert_close(got, exp)
-    del got
+    del got, filler
     assert torch.equal(call(), exp)

@@ -247,8 +247,9 @@ def _forward(q: Tensor, k: Tensor, v: Tensor, cu_seqlens_q: Optional[Tensor], cu
             try:
                 ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
             except torch.OutOfMemoryError:
-                ws, nbytes = None, 0  # the keys then stay whole
-            _lib.check(L.mykfa_fwd_grown(ctypes.byref(p), 0, _ptr(ws), nbytes, _stream(dev)))
+                ws = None  # the keys then stay whole
+            _lib.check(L.mykfa_fwd(ctypes.byref(p), _stream(dev)) if ws is None else
+                       L.mykfa_fwd_ws(ctypes.byref(p), ws.data_ptr(), nbytes, _stream(dev)))
         else:
             _lib.check(L.mykfa_fwd(ctypes.byref(p), _stream(dev)))
     return out, lse

@@ -195,6 +195,22 @@ def test_grown_lengths_need_the_cached_ones(L):
     assert L.mykfa_fwd_grown(ctypes.byref(p), 4, None, 0, None) == _lib.OK  # nothing to do
 
 
+def test_split_forward_checks_its_workspace(L):
+    p = good_fwd()
+    p.batch, p.num_heads, p.num_kv_heads, p.head_dim, p.max_seqlen_q, p.max_seqlen_k = 1, 16, 4, 128, 389, 8192
+    for t, h, n in (("q", 16, 389), ("k", 4, 8192), ("v", 4, 8192), ("o", 16, 389)):
+        setattr(p, f"{t}_batch_stride", n * h * 128)
+        setattr(p, f"{t}_token_stride", h * 128)
+        setattr(p, f"{t}_head_stride", 128)
+    p.lse_head_stride = 389
+    need = L.mykfa_fwd_workspace_size(ctypes.byref(p))
+    assert need == 8 * 16 * 389 * 130 * 4  # eight slots a block, O and (m, l) in fp32
+    assert L.mykfa_fwd_ws(ctypes.byref(p), None, 0, None) == _lib.ERR_WORKSPACE
+    assert L.mykfa_fwd_ws(ctypes.byref(p), 0x10000, need - 1, None) == _lib.ERR_WORKSPACE
+    assert L.mykfa_fwd_grown(ctypes.byref(p), 0, 0x10000, need - 1, None) == _lib.ERR_WORKSPACE
+    assert L.mykfa_fwd_ws(ctypes.byref(p), 0x10008, need, None) == _lib.ERR_INVALID
+
+
 def test_decode_split_heuristic(L):
     # Full 16K caches of a 64-sequence batch: ~1408 keys per split, 12 splits, for one query of
     # a 4-head group and for the 4-query draft alike.

@@ -1,7 +1,7 @@
 """CPU oracle for the FlashAttention path — TEST INFRASTRUCTURE ONLY.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import this module,
-and only as the checker (or the timed CPU baseline). The product path
+and only as the oracle (or the timed CPU baseline). The product path
 (myk_llm_amd.flash_attn) never calls it and fails loudly without the HIP library.
 
 Restated from the reference (never imported):

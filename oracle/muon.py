@@ -1,6 +1,6 @@
 """CPU oracle for Muon's batched SYRK and Newton-Schulz iteration — TEST INFRASTRUCTURE ONLY.
 
-Only tests/ and bench.py's cpu_baseline leg may import this module, as the checker. The
+Only tests/ and bench.py's cpu_baseline leg may import this module, as the oracle. The
 product path (myk_llm_amd.muon) never calls it and fails loudly without the HIP library.
 
 Restated from the reference (never imported):
